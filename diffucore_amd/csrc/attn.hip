@@ -890,28 +890,6 @@ constexpr int64_t WIDE_MAX_VSL = (int64_t)1 << 23;
 // 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
 #define DC_ATTN_WAIT_VMCNT(n_) __builtin_amdgcn_s_waitcnt(((n_) & 15) | (((n_) >> 4) << 14) | (7 << 4) | (15 << 8))
 
-typedef __attribute__((address_space(3))) void* lds_void_ptr_t;
-
-// One DMA of 16 bytes per lane from global memory into LDS
-// (global_load_lds_dwordx4 from the wave-uniform address `base` plus the
-// lane's byte offset `off`; lane i's bytes land at m0 + 16 i, `lds` being the
-// wave's LDS destination, a byte address in the LDS address space). Inline
-// asm, so the compiler's wait-count pass does not see an LDS store: it cannot
-// tell the ring stages apart and otherwise waits for every DMA in flight
-// (vmcnt(0)) before some of the next tile's LDS reads, which measured 3% of
-// the kernel's time at the FLUX shape. The kernel orders each stage's writes
-// and reads itself, by vmcnt waits and barriers.
-__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base),
-               "{m0}"(__builtin_amdgcn_readfirstlane(lds))
-               : "memory");
-}
-
-// LDS byte address of a pointer into a __shared__ array.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)reinterpret_cast<uintptr_t>((lds_void_ptr_t)(const_cast<void*>(p)));
-}
-
 // The 2 Dp / 32 K operands (k-step ks, key block kb) of one 64-key tile from a
 // swizzled K stage; kfo[ks] is the lane's byte offset of its 16-byte chunk for
 // k-step ks (row l32).

@@ -121,6 +121,29 @@ __device__ __forceinline__ void static_for(F&& f) {
   StaticFor<0, N>::run(f);
 }
 
+// ---------------------------------------------------------------- global memory -> LDS
+
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+
+// LDS byte address of a pointer into a __shared__ array.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)reinterpret_cast<uintptr_t>((lds_void_ptr)(const_cast<void*>(p)));
+}
+
+// One DMA of 16 bytes per lane from global memory into LDS
+// (global_load_lds_dwordx4 from the wave-uniform address `base` plus the
+// lane's byte offset `off`; lane i's bytes land at m0 + 16 i, `lds` being the
+// wave's LDS destination, a byte address in the LDS address space). Inline
+// asm, so the compiler's wait-count pass does not see an LDS store: it cannot
+// tell the stages of a ring apart and otherwise waits for every DMA in flight
+// (vmcnt(0)) before some of the next stage's LDS reads. The kernels order each
+// stage's writes and reads themselves, by vmcnt waits and barriers.
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base),
+               "{m0}"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory");
+}
+
 // ---------------------------------------------------------------- wave reductions
 
 __device__ __forceinline__ float wave_max(float v) {

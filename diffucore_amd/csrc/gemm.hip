@@ -10,21 +10,24 @@
 // channels n per register quad (8- or 16-byte stores in the epilogue).
 //   workgroup tile  BN x BM = (32*WN*FN) x (32*WM*FM), WN x WM waves
 //   wave tile       (32*FN) x (32*FM) = FN x FM MFMA blocks of 32 x 32
-//   k depth         128 bytes per LDS stage, two stages
-// Four instantiations: 256 x 256 tiles on 8 waves (2 along n x 4 along m,
-// each 128 x 64), 192 x 256 on 8 waves (each 96 x 64), 192 x 128 on 4 waves
-// (each 96 x 64) and 128 x 128 on 4 waves (each 64 x 64); pick_tile chooses
-// by how full the last round of tiles is.
-// 256 x 256 tiles with K % 256 == 0 go to w8a8_gemm_dma_kernel instead (4
-// waves of 128 x 128, operands loaded straight into LDS; described there).
-// Pipeline per 128-byte k tile (4 MFMA k-steps): operand fragments for the
-// next k-step are read from LDS while the current one's MFMAs run; the next
-// tile, staged in registers, is written to the other LDS stage after the first
-// k-step; the tile after that is fetched from global memory after the second.
-// LDS rows are padded from 128 to 144 bytes so the 32 rows an operand read
-// touches spread over all banks, and every read address is a per-lane base
-// plus an immediate. Tiles are ordered so each XCD (8 per device; the hardware
-// deals workgroups round-robin over them) works a contiguous, L2-friendly range.
+// Two kernels:
+//   w8a8_gemm_dma_kernel  K % 64 == 0 (every layer width of the SD1.5, SDXL
+//     and FLUX models): operands loaded straight into an LDS ring; seven tiles
+//     from 64 x 64 to 256 x 256, chosen by pick_dma.
+//   w8a8_gemm_kernel      the other K (multiples of 16) and row strides past
+//     the DMA's 32-bit offsets: 128 k-bytes per LDS stage, two stages; 256 x
+//     256 tiles on 8 waves (2 along n x 4 along m, each 128 x 64), 192 x 256
+//     on 8 waves (each 96 x 64), 192 x 128 on 4 waves (each 96 x 64) and
+//     128 x 128 on 4 waves (each 64 x 64), chosen by plan_tile. Per 128-byte
+//     k tile (4 MFMA k-steps): operand fragments for the next k-step are read
+//     from LDS while the current one's MFMAs run; the next tile, staged in
+//     registers, is written to the other LDS stage after the first k-step;
+//     the tile after that is fetched from global memory after the second.
+//     LDS rows are padded from 128 to 144 bytes so the 32 rows an operand
+//     read touches spread over all banks, and every read address is a
+//     per-lane base plus an immediate.
+// Tiles are ordered so each XCD (8 per device; the hardware deals workgroups
+// round-robin over them) works a contiguous, L2-friendly range.
 #include "common.h"
 
 #include <atomic>
@@ -371,109 +374,8 @@ struct EpiRegs {
   }
 };
 
-// Epilogue of one wave's full 128 (n) x 128 (m) block through LDS: the output
-// values go to the wave's own 32 KB of LDS (`stage`, free after the main
-// loop), row m at 128 * (output bytes) per row, 16-byte chunk c of row r at
-// chunk c ^ (r % 16); then each row leaves as one contiguous run, 16 bytes per
-// lane (4 rows per store instruction for 16-bit outputs, 2 for 32-bit). The
-// MFMA layout would otherwise store 8 or 16 bytes into each of 32 rows per
-// instruction. 32-bit outputs take two passes of 64 rows. A lane reads back
-// what other lanes of its wave wrote: the wavefront fences and barrier
-// between the two halves keep the compiler from moving LDS accesses across.
-// RES: the gated residual. The residual chunks the lane stores go through a
-// ring of RRING registers, loaded RRING stores ahead: the first RRING before
-// the pass converts (they land meanwhile), each later one as its slot frees
-// (a whole pass at once would spill). The lane's gate values come from g_l.
-template <int OUT_DT, int BIAS_DT, bool RES = false>
-__device__ __forceinline__ void store_tile_lds(const v16i (&acc)[4][4], const GemmArgs& p, int m0, int n0, int nb,
-                                               int mb, const float* sw_l, const float* b_l, const float* sx_l, int hf,
-                                               int l32, int lane, uint8_t* stage, const float* g_l = nullptr) {
-  constexpr int OB = (OUT_DT == DC_F16 || OUT_DT == DC_BF16) ? 2 : 4;
-  constexpr int ROWB = 128 * OB;   // staged row bytes
-  constexpr int CH = ROWB / 16;    // 16-byte chunks per row
-  constexpr int JP = 8 / OB;       // 32-row m blocks per pass
-  constexpr int RPI = 64 / CH;     // rows per store instruction
-  constexpr int NIT = 32 * JP / RPI;   // store instructions per pass
-  constexpr int RRING = 8;             // residual chunks in flight per lane
-  constexpr bool HB = BIAS_DT != DC_NONE;
-  const int c = lane % CH;
-  float sxm[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) sxm[j] = OUT_DT != DC_I32 ? sx_l[mb + 32 * j + l32] : 0.0f;
-  float gv[RES ? 16 / OB : 1];
-  if constexpr (RES) {
-#pragma unroll
-    for (int e = 0; e < 16 / OB; ++e) gv[e] = g_l[nb + (16 / OB) * c + e];
-  }
-#pragma unroll
-  for (int j0 = 0; j0 < 4; j0 += JP) {
-    uint4 rres[RES ? RRING : 1];
-    const uint8_t* rrow = RES ? static_cast<const uint8_t*>(p.res) + (n0 + nb) * OB + 16 * c : nullptr;
-    auto rload = [&](int k) __attribute__((always_inline)) {
-      return *reinterpret_cast<const uint4*>(rrow + (int64_t)(m0 + mb + 32 * j0 + RPI * k + lane / CH) * p.ldr * OB);
-    };
-    if constexpr (RES) {
-#pragma unroll
-      for (int k = 0; k < RRING; ++k) rres[k] = rload(k);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int nl = nb + 32 * i + 8 * g + 4 * hf;
-        float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f), b4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (OUT_DT != DC_I32) s4 = *reinterpret_cast<const float4*>(sw_l + nl);
-        if constexpr (HB) b4 = *reinterpret_cast<const float4*>(b_l + nl);
-#pragma unroll
-        for (int jj = 0; jj < JP; ++jj) {
-          const int j = j0 + jj, r = 32 * jj + l32;
-          uint8_t* row = stage + r * ROWB;
-          const int av[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-          if constexpr (OUT_DT == DC_I32) {
-            const int c = 8 * i + 2 * g + hf;
-            *reinterpret_cast<int4*>(row + 16 * (c ^ (r & 15))) = make_int4(av[0], av[1], av[2], av[3]);
-          } else if constexpr (OUT_DT == DC_F32) {
-            const int c = 8 * i + 2 * g + hf;
-            const float y0 = epi_pre<OUT_DT, HB>(av[0], sxm[j], s4.x, b4.x);
-            const float y1 = epi_pre<OUT_DT, HB>(av[1], sxm[j], s4.y, b4.y);
-            const float y2 = epi_pre<OUT_DT, HB>(av[2], sxm[j], s4.z, b4.z);
-            const float y3 = epi_pre<OUT_DT, HB>(av[3], sxm[j], s4.w, b4.w);
-            *reinterpret_cast<float4*>(row + 16 * (c ^ (r & 15))) = make_float4(y0, y1, y2, y3);
-          } else {
-            const int c = 4 * i + g;
-            const uint32_t lo = epi_pair<OUT_DT, HB>(av[0], av[1], sxm[j], s4.x, s4.y, b4.x, b4.y);
-            const uint32_t hi = epi_pair<OUT_DT, HB>(av[2], av[3], sxm[j], s4.z, s4.w, b4.z, b4.w);
-            *reinterpret_cast<uint2*>(row + 16 * (c ^ (r & 15)) + 8 * hf) = make_uint2(lo, hi);
-          }
-        }
-      }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int k = 0; k < NIT; ++k) {
-      const int r = RPI * k + lane / CH;
-      uint4 v = *reinterpret_cast<const uint4*>(stage + r * ROWB + 16 * (c ^ (r & 15)));
-      if constexpr (RES) {
-        const uint4 rk = rres[k % RRING];
-        if (k + RRING < NIT) rres[k % RRING] = rload(k + RRING);
-        v = gated_chunk<OUT_DT>(v, rk, gv);
-      }
-      const int64_t m = m0 + mb + 32 * j0 + r;
-      uint8_t* dst = static_cast<uint8_t*>(p.out) + (m * p.ldo + n0 + nb) * OB + 16 * c;
-      *reinterpret_cast<uint4*>(dst) = v;
-    }
-    if constexpr (JP < 4) {
-      // the next pass overwrites what this one read back
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-  }
-}
-
-// Epilogue of one wave's full (32 FN) n x (32 FM) m block through LDS, for the
-// register-staged kernel: the wave's outputs go to its own WAVE_BYTES of the
+// Epilogue of one wave's full (32 FN) n x (32 FM) m block through LDS: the
+// wave's outputs go to its own WAVE_BYTES of the
 // LDS stages (free after the main loop), row m at a pitch of its bytes plus
 // 16 (the padding spreads a 16-byte write of 16 consecutive rows over all
 // banks), JP 32-row m blocks per pass; then each row leaves as one contiguous
@@ -482,10 +384,15 @@ __device__ __forceinline__ void store_tile_lds(const v16i (&acc)[4][4], const Ge
 // store_tile. A lane reads back what other lanes of its wave wrote: the
 // wavefront fences and barrier keep the compiler from moving LDS accesses
 // across.
-template <int OUT_DT, int BIAS_DT, int FN, int FM, int WAVE_BYTES>
+// RES: the gated residual. The residual chunks a lane stores are loaded
+// before their pass converts, so that they land meanwhile; the lane's gate
+// values (its chunk's column is the same in every store: CH divides 64) come
+// from g_l.
+template <int OUT_DT, int BIAS_DT, int FN, int FM, int WAVE_BYTES, bool RES = false>
 __device__ __forceinline__ void store_tile_staged(const v16i (&acc)[FN][FM], const GemmArgs& p, int m0, int n0, int nb,
                                                   int mb, const float* sw_l, const float* b_l, const float* sx_l,
-                                                  int hf, int l32, int lane, uint8_t* stage) {
+                                                  int hf, int l32, int lane, uint8_t* stage,
+                                                  const float* g_l = nullptr) {
   constexpr int OB = (OUT_DT == DC_F16 || OUT_DT == DC_BF16) ? 2 : 4;
   constexpr int ROWB = 32 * FN * OB;   // output row bytes of the block
   constexpr int RP = ROWB + 16;        // staged row pitch
@@ -495,11 +402,24 @@ __device__ __forceinline__ void store_tile_staged(const v16i (&acc)[FN][FM], con
   static_assert(32 * RP <= WAVE_BYTES, "one 32-row block must fit the wave's LDS share");
   static_assert((32 * JP * CH) % 64 == 0, "a pass must be whole store instructions");
   constexpr bool HB = BIAS_DT != DC_NONE;
+  static_assert(!RES || 64 % CH == 0, "a lane's gate column must not depend on the store");
   float sxm[FM];
 #pragma unroll
   for (int j = 0; j < FM; ++j) sxm[j] = OUT_DT != DC_I32 ? sx_l[mb + 32 * j + l32] : 0.0f;
+  float gv[RES ? 16 / OB : 1];
+  if constexpr (RES) {
+#pragma unroll
+    for (int e = 0; e < 16 / OB; ++e) gv[e] = g_l[nb + (16 / OB) * (lane % CH) + e];
+  }
 #pragma unroll
   for (int j0 = 0; j0 < FM; j0 += JP) {
+    uint4 rres[RES ? NIT : 1];
+    if constexpr (RES) {
+      const uint8_t* rrow = static_cast<const uint8_t*>(p.res) + (n0 + nb) * OB + 16 * (lane % CH);
+#pragma unroll
+      for (int k = 0; k < NIT; ++k)
+        rres[k] = *reinterpret_cast<const uint4*>(rrow + (int64_t)(m0 + mb + 32 * j0 + (64 * k + lane) / CH) * p.ldr * OB);
+    }
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
@@ -534,7 +454,8 @@ __device__ __forceinline__ void store_tile_staged(const v16i (&acc)[FN][FM], con
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
       const int idx = 64 * k + lane, r = idx / CH, c = idx % CH;
-      const uint4 v = *reinterpret_cast<const uint4*>(stage + r * RP + 16 * c);
+      uint4 v = *reinterpret_cast<const uint4*>(stage + r * RP + 16 * c);
+      if constexpr (RES) v = gated_chunk<OUT_DT>(v, rres[k], gv);
       const int64_t m = m0 + mb + 32 * j0 + r;
       *reinterpret_cast<uint4*>(static_cast<uint8_t*>(p.out) + (m * p.ldo + n0 + nb) * OB + 16 * c) = v;
     }
@@ -727,176 +648,202 @@ __global__ void __launch_bounds__(T::NT, 1) w8a8_gemm_kernel(GemmArgs p) {
 
 // ---------------------------------------------------------------- DMA-fed kernel
 //
-// 256 x 256 tiles on 4 waves (2 along n x 2 along m, each 128 x 128 = 4 x 4
-// MFMA blocks, accumulators in AGPRs, one wave per SIMD). Operands go from
-// global memory straight into LDS (global_load_lds_dwordx4: lane i of a wave
-// writes bytes 16 i .. 16 i + 15 after the wave's base) through 4 stages of 64
-// k-bytes, up to 4 stages ahead of the MFMAs, so no registers stage them. A stage is
-// W [256 rows x 64 B] then A [256 rows x 64 B], unpadded; the 16-byte chunk c
-// of row r sits at chunk c ^ ((r / 4) % 4), which spreads the 16 rows a
-// fragment read serves per cycle over all banks. One barrier per stage, half
-// way through it: every wave has waited for its own loads of the next stage
-// (vmcnt) and for its own fragment reads of the current one (lgkmcnt), so
-// after the barrier the next stage is complete and the current stage's buffer
-// is free for the loads 4 stages ahead.
-// Needs K % 256 == 0 (whole stages, 4 per trip of the unrolled loop) and
-// 256 * ldw, 256 * lda below 2^31.
-constexpr int DBK = 64;                      // k bytes per stage
-constexpr int DSTAGE = (256 + 256) * DBK;    // 32 KB
-constexpr int DMA_LOADS_PER_STAGE = 8;       // per wave: 4 KB of W + 4 KB of A
+// Operands go from global memory straight into LDS (global_load_lds_dwordx4:
+// lane i of a wave writes bytes 16 i .. 16 i + 15 after the wave's base), so no
+// registers stage them, through a ring of S stages of KB k-bytes: W [BN rows x
+// KB], then A [BM rows x KB], unpadded. KB = 128: every DMA reads whole
+// 128-byte lines (8 rows per instruction). At 64-byte rows (the tile then
+// loads each line in two visits) the 256 x 256 tiles measured 306.8 us at
+// 4608 x 3072 -> 21504 against 280.8 here, 162.4 against 141.6 at 4096 x 3072
+// -> 12288, 220.0 against 192.8 at 4608 x 15360 -> 3072. KB = 64 is for K =
+// 64 (mod 128) only.
+// Chunk c (16 bytes) of row r sits at c ^ ((r / 2) % 8) (KB = 128) or c ^
+// ((r / 4) % 4) (KB = 64): the 16 rows a fragment read serves per cycle cover
+// all banks.
+// One barrier per stage, before its last k-step: every wave has waited for
+// its own loads of the next stage (vmcnt) and for its own fragment reads of
+// the current one (lgkmcnt), so after the barrier the next stage is complete
+// and the current stage's buffer is free for the loads S stages ahead; the
+// last k-step then runs while the first fragments of the next stage are read.
+// Fragments are read one k-step ahead throughout. The last S stages issue no
+// loads and wait by what is left in flight.
+// Needs K % KB == 0 and 256 * ldw, 256 * lda below 2^31.
+template <int WN_, int WM_, int FN_, int FM_, int S_, int KB_, int OCC_>
+struct DmaTile {
+  static constexpr int WN = WN_, WM = WM_, FN = FN_, FM = FM_;   // waves along n and m, MFMA blocks per wave
+  static constexpr int S = S_, KB = KB_;
+  static constexpr int OCC = OCC_;                               // waves per SIMD the registers must allow
+  static constexpr int NW = WN * WM, NT = 64 * NW;
+  static constexpr int BN = 32 * WN * FN, BM = 32 * WM * FM;
+  static constexpr int STAGE = (BN + BM) * KB;
+  static constexpr int CPR = KB / 16, RPD = 64 / CPR;            // chunks per row, rows per DMA instruction
+  static constexpr int LW = BN / RPD / NW, LA = BM / RPD / NW;   // DMA instructions per wave and stage
+  static constexpr int lds_bytes(bool res) { return S * STAGE + ((res ? 3 : 2) * BN + BM) * 4; }
+  static_assert(KB == 64 || KB == 128, "stage depth");
+  static_assert(BN % (RPD * NW) == 0 && BM % (RPD * NW) == 0, "whole DMA instructions per wave");
+  static_assert(BN <= NT && BM <= NT, "EpiRegs holds one epilogue-vector entry per thread");
+  static_assert(lds_bytes(true) <= 160 * 1024, "LDS per CU");
+};
 
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
+// The tiles (n x m; LDS per workgroup), each the fastest of the sizes that
+// pick_dma gives it; figures there.
+typedef DmaTile<4, 2, 2, 4, 2, 128, 2> Dma256x256;    // 8 waves of 64 x 128, 128 KB
+typedef DmaTile<2, 4, 3, 2, 2, 128, 2> Dma192x256;    // 8 waves of 96 x 64, 112 KB
+typedef DmaTile<2, 2, 2, 2, 2, 128, 2> Dma128x128;    // 4 waves of 64 x 64, 64 KB: 2 workgroups per CU
+typedef DmaTile<2, 4, 2, 1, 3, 128, 2> Dma128x128d;   // 8 waves of 64 x 32, 96 KB, 3 stages: 1 per CU
+typedef DmaTile<2, 4, 1, 1, 3, 128, 4> Dma64x128;     // 8 waves of 32 x 32, 72 KB: 2 per CU
+typedef DmaTile<2, 2, 1, 1, 3, 128, 3> Dma64x64;      // 4 waves of 32 x 32, 48 KB: 3 per CU
+typedef DmaTile<2, 2, 2, 2, 3, 64, 3> Dma128x128k;    // 4 waves of 64 x 64, 48 KB, 64-byte stages: 3 per CU
 
-// vmcnt(n) with the other counters left unconstrained, and vmcnt(n) together
-// with lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4,
-// lgkmcnt 11:8)
-#define DC_WAIT_VMCNT(n_) __builtin_amdgcn_s_waitcnt(((n_) & 15) | (((n_) >> 4) << 14) | (7 << 4) | (15 << 8))
-#define DC_WAIT_VMCNT_LGKM0(n_) __builtin_amdgcn_s_waitcnt(((n_) & 15) | (((n_) >> 4) << 14) | (7 << 4))
+// vmcnt(n) with the other counters left unconstrained, and lgkmcnt(0) (gfx9
+// encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt has 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+__device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
 // RES: with the gated residual of dc_w8a8_gemm_grouped_gated.
-template <int OUT_DT, int BIAS_DT, bool RES = false>
-__global__ void __launch_bounds__(256, 1) w8a8_gemm_dma_kernel(GemmArgs p, GroupArgs g) {
-  constexpr int BN = 256, BM = 256, FN = 4, FM = 4;
-  __shared__ __attribute__((aligned(1024))) uint8_t st0[DSTAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st1[DSTAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st2[DSTAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st3[DSTAGE];
-  __shared__ __attribute__((aligned(16))) float epi_v[(RES ? 3 : 2) * BN + BM];
+template <class T, int OUT_DT, int BIAS_DT, bool RES = false>
+__global__ void __launch_bounds__(T::NT, T::OCC) w8a8_gemm_dma_kernel(GemmArgs p, GroupArgs g) {
+  constexpr int FN = T::FN, FM = T::FM, BN = T::BN, BM = T::BM, S = T::S, KB = T::KB, L = T::LW + T::LA;
+  constexpr int NKS = KB / 32;   // MFMA k-steps per stage
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int l32 = lane & 31, hf = lane >> 5;
-  const int wn = w & 1, wm = w >> 1;
+  const int wn = w % T::WN, wm = w / T::WN;
   int m0, n0;
   if (g.ngroup > 0) group_origin(p, g, BM, BN, m0, n0);
   else tile_origin(p, BM, BN, m0, n0);
 
-  float* sw_l = epi_v;
-  float* b_l = epi_v + BN;
-  float* sx_l = epi_v + 2 * BN;
-  float* g_l = RES ? epi_v + 2 * BN + BM : nullptr;
+  float* sw_l = reinterpret_cast<float*>(smem + S * T::STAGE);
+  float* b_l = sw_l + BN;
+  float* sx_l = b_l + BN;
+  float* g_l = RES ? sx_l + BM : nullptr;
   // issued ahead of the operand loads; staged in LDS after the main loop
   const EpiRegs ev = EpiRegs::load<OUT_DT, BIAS_DT, RES>(p, m0, n0, BM, BN, t);
 
-  // DMA sources: wave w loads 1 KB blocks j = w + 4 u (rows 16 j .. 16 j + 15)
-  // of W and of A; lane i covers row 16 j + i / 4, logical chunk
-  // (i % 4) ^ ((i / 16) % 4) (its physical chunk is i % 4).
-  // (byte offsets from the tile's first W / A row; rows past N / M are clamped)
-  const int drow = lane >> 2, dchunk = (lane & 3) ^ ((lane >> 4) & 3);
+  // DMA sources: wave w loads RPD-row blocks w + NW u of W and of A; lane i
+  // covers row i / CPR of its block, physical chunk i % CPR (byte offsets from
+  // the tile's first W / A row; rows past N / M are clamped)
+  auto swz = [](int r) { return KB == 64 ? (r >> 2) & 3 : (r >> 1) & 7; };
+  const int drow = lane / T::CPR, dchunk = lane % T::CPR;
   const int8_t* wtile = p.w + (int64_t)n0 * p.ldw;
   const int8_t* atile = p.a + (int64_t)m0 * p.lda;
-  uint32_t woff[4], aoff[4];   // unsigned: a scalar base plus a 32-bit lane offset
+  uint32_t woff[T::LW], aoff[T::LA];   // unsigned: a scalar base plus a 32-bit lane offset
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int r = 16 * (w + 4 * u) + drow;
-    woff[u] = (uint32_t)((min(n0 + r, p.N - 1) - n0) * (int)p.ldw + 16 * dchunk);
-    aoff[u] = (uint32_t)((min(m0 + r, p.M - 1) - m0) * (int)p.lda + 16 * dchunk);
+  for (int u = 0; u < T::LW; ++u) {
+    const int r = T::RPD * (w + T::NW * u) + drow;
+    woff[u] = (uint32_t)((min(n0 + r, p.N - 1) - n0) * (int)p.ldw + 16 * (dchunk ^ swz(r)));
   }
-  const int nk = p.K / DBK;   // a multiple of 4
-  // stage kt's loads; stages past the end re-read the last one (kept in bounds;
-  // their data is never used)
-#define DMA_STAGE(buf_, kt_)                                                                             \
-  {                                                                                                      \
-    const int k0_ = min((kt_), nk - 1) * DBK;                                                            \
-    _Pragma("unroll") for (int u = 0; u < 4; ++u)                                                        \
-        __builtin_amdgcn_global_load_lds((wtile + k0_) + woff[u], (lds_void_ptr)((buf_) + 1024 * (w + 4 * u)), 16, 0, 0); \
-    _Pragma("unroll") for (int u = 0; u < 4; ++u)                                                        \
-        __builtin_amdgcn_global_load_lds((atile + k0_) + aoff[u], (lds_void_ptr)((buf_) + 16384 + 1024 * (w + 4 * u)), 16, 0, 0); \
+#pragma unroll
+  for (int u = 0; u < T::LA; ++u) {
+    const int r = T::RPD * (w + T::NW * u) + drow;
+    aoff[u] = (uint32_t)((min(m0 + r, p.M - 1) - m0) * (int)p.lda + 16 * (dchunk ^ swz(r)));
   }
+  const uint32_t lds0 = lds_addr(smem) + 1024 * w;
+  const int nk = p.K / KB;
+  auto issue = [&](int kt, int slot) __attribute__((always_inline)) {
+    const uint32_t d = lds0 + slot * T::STAGE;
+    const int k0 = kt * KB;
+#pragma unroll
+    for (int u = 0; u < T::LW; ++u) dma16(wtile + k0, woff[u], d + 1024 * T::NW * u);
+#pragma unroll
+    for (int u = 0; u < T::LA; ++u) dma16(atile + k0, aoff[u], d + BN * KB + 1024 * T::NW * u);
+  };
 
-  // fragment reads: W rows wn*128 + 32 i + l32, A rows wm*128 + 32 j + l32; k-step
-  // ks reads logical chunk 2 ks + hf, physical (2 ks + hf) ^ ((l32 / 4) % 4)
-  const int swz = (l32 >> 2) & 3;
-  const int wrow = (wn * 128 + l32) * DBK, arow = 16384 + (wm * 128 + l32) * DBK;
-  const int kc0 = 16 * (hf ^ swz), kc1 = 16 * ((2 + hf) ^ swz);
+  // fragment reads: W rows wn * 32 FN + 32 i + l32, A rows wm * 32 FM + 32 j +
+  // l32; k-step ks reads logical chunk 2 ks + hf
+  const int sx = swz(l32);
+  const int wrow = (wn * 32 * FN + l32) * KB, arow = BN * KB + (wm * 32 * FM + l32) * KB;
+  int kc[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) kc[ks] = 16 * ((2 * ks + hf) ^ sx);
   v16i acc[FN][FM];
 #pragma unroll
   for (int i = 0; i < FN; ++i)
 #pragma unroll
     for (int j = 0; j < FM; ++j) acc[i][j] = v16i{0};
   v4i wf[2][FN], af[2][FM];
-#define DMA_FRAGS(b_, buf_, kc_)                                                                         \
-  {                                                                                                      \
-    _Pragma("unroll") for (int i = 0; i < FN; ++i)                                                       \
-        wf[b_][i] = *reinterpret_cast<const v4i*>((buf_) + wrow + 2048 * i + (kc_));                     \
-    _Pragma("unroll") for (int j = 0; j < FM; ++j)                                                       \
-        af[b_][j] = *reinterpret_cast<const v4i*>((buf_) + arow + 2048 * j + (kc_));                     \
-  }
-#define DMA_MFMAS(b_)                                                                                    \
-  _Pragma("unroll") for (int i = 0; i < FN; ++i)                                                         \
-  _Pragma("unroll") for (int j = 0; j < FM; ++j)                                                         \
-      acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[b_][i], af[b_][j], acc[i][j], 0, 0, 0);
+  auto frags = [&](int buf, int slot, int ks) __attribute__((always_inline)) {
+    const uint8_t* b = smem + slot * T::STAGE + kc[ks];
+#pragma unroll
+    for (int i = 0; i < FN; ++i) wf[buf][i] = *reinterpret_cast<const v4i*>(b + wrow + 32 * KB * i);
+#pragma unroll
+    for (int j = 0; j < FM; ++j) af[buf][j] = *reinterpret_cast<const v4i*>(b + arow + 32 * KB * j);
+  };
+  auto mfmas = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[buf][i], af[buf][j], acc[i][j], 0, 0, 0);
+  };
+  // waits until at most the newest n stages of this wave's loads are in flight
+  auto wait_left = [&](int n) __attribute__((always_inline)) {
+    static_assert(S <= 4, "wait_left handles up to 3 stages in flight");
+    if (S > 3 && n >= 3) wait_vmcnt<3 * L>();
+    else if (S > 2 && n >= 2) wait_vmcnt<2 * L>();
+    else if (n >= 1) wait_vmcnt<L>();
+    else wait_vmcnt<0>();
+  };
+  // the barrier that ends the waits above: no LDS access moves across it
+  auto sync = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-  DMA_STAGE(st0, 0);
-  DMA_STAGE(st1, 1);
-  DMA_STAGE(st2, 2);
-  DMA_STAGE(st3, 3);
-  DC_WAIT_VMCNT(3 * DMA_LOADS_PER_STAGE);
-  __builtin_amdgcn_s_barrier();
-  DMA_FRAGS(0, st0, kc0);
-
-  // Iteration kt (stage buffer cur = kt % 4): k-step 0 runs on fragments read
-  // earlier while k-step 1's are read from cur; then the wave waits for its
-  // loads of stage kt + 1 and for its reads of cur, the barrier makes stage
-  // kt + 1 complete and cur free, the loads of stage kt + 4 go into cur, and
-  // k-step 1 runs while the first fragments of stage kt + 1 are read.
-#define DMA_ITER(kt_, cur_, nxt_)                                                                        \
-  {                                                                                                      \
-    DMA_FRAGS(1, cur_, kc1);                                                                             \
-    DMA_MFMAS(0);                                                                                        \
-    /* one MFMA first: its wait covers only the fragments it uses */                                     \
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                   \
-    _Pragma("unroll") for (int z = 0; z < 8; ++z) {                                                      \
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                                                 \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                 \
-    }                                                                                                    \
-    __builtin_amdgcn_sched_group_barrier(0x008, 7, 0);                                                   \
-    __builtin_amdgcn_sched_barrier(0);                                                                   \
-    DC_WAIT_VMCNT_LGKM0(2 * DMA_LOADS_PER_STAGE);                                                        \
-    __builtin_amdgcn_s_barrier();                                                                        \
-    __builtin_amdgcn_sched_barrier(0);                                                                   \
-    DMA_STAGE(cur_, (kt_) + 4);                                                                          \
-    DMA_FRAGS(0, nxt_, kc0);                                                                             \
-    DMA_MFMAS(1);                                                                                        \
-    /* the next fragment reads with the first 8 MFMAs (they return during the  \
-       last 8, so the next iteration's first MFMA does not wait on them), the  \
-       stage's loads with the last 8 */                                                                  \
-    _Pragma("unroll") for (int z = 0; z < 8; ++z) {                                                      \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                 \
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                                                 \
-    }                                                                                                    \
-    _Pragma("unroll") for (int z = 0; z < 8; ++z) {                                                      \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                 \
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                                                 \
-    }                                                                                                    \
-    __builtin_amdgcn_sched_barrier(0);                                                                   \
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < nk) issue(s, s);
+  wait_left(min(nk, S) - 1);
+  sync();
+  frags(0, 0, 0);
+  int kt = 0, slot = 0;
+  // stage kt in `slot`; MORE: stage kt + S exists
+  auto stage = [&](auto more) __attribute__((always_inline)) {
+    constexpr bool MORE = decltype(more)::value;
+#pragma unroll
+    for (int ks = 0; ks < NKS - 1; ++ks) {
+      frags((ks + 1) & 1, slot, ks + 1);
+      mfmas(ks & 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int next = slot == S - 1 ? 0 : slot + 1;
+    if constexpr (MORE) wait_vmcnt<(S - 2) * L>();
+    else wait_left(nk - 2 - kt);
+    wait_lgkmcnt0();
+    sync();
+    if constexpr (MORE) issue(kt + S, slot);
+    frags(0, next, 0);
+    mfmas(1);
+    __builtin_amdgcn_sched_barrier(0);
+    slot = next;
+    ++kt;
+  };
+  static_assert(NKS % 2 == 0, "a stage starts on fragment buffer 0");
+  while (kt + S < nk) stage(std::true_type{});
+  while (kt + 1 < nk) stage(std::false_type{});
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    if (ks + 1 < NKS) frags((ks + 1) & 1, slot, ks + 1);
+    mfmas(ks & 1);
   }
-  for (int kt = 0; kt < nk; kt += 4) {
-    DMA_ITER(kt, st0, st1);
-    DMA_ITER(kt + 1, st1, st2);
-    DMA_ITER(kt + 2, st2, st3);
-    DMA_ITER(kt + 3, st3, st0);
-  }
-#undef DMA_ITER
-#undef DMA_MFMAS
-#undef DMA_FRAGS
-#undef DMA_STAGE
-  // no load may still be writing this workgroup's LDS when it ends
-  DC_WAIT_VMCNT(0);
+  // (every load was waited for before the last stage was read)
   ev.stage<OUT_DT, BIAS_DT, RES>(BM, BN, t, sw_l, b_l, sx_l, g_l);
-  __syncthreads();   // the epilogue vectors are in LDS; every wave is done reading the stage buffers
+  __syncthreads();   // the epilogue vectors are in LDS; every wave is done reading the ring
 
-  if (p.vec16 && m0 + BM <= p.M && n0 + BN <= p.N) {
-    uint8_t* stg = w == 0 ? st0 : (w == 1 ? st1 : (w == 2 ? st2 : st3));
-    store_tile_lds<OUT_DT, BIAS_DT, RES>(acc, p, m0, n0, wn * 128, wm * 128, sw_l, b_l, sx_l, hf, l32, lane, stg,
-                                         g_l);
-  } else {
-    store_tile<OUT_DT, BIAS_DT, FN, FM, RES>(acc, p, m0, n0, wn * 32 * FN, wm * 32 * FM, BM, BN, sw_l, b_l, sx_l,
-                                             hf, l32, g_l);
-  }
+  constexpr int WAVE_BYTES = S * T::STAGE / T::NW / 16 * 16;
+  if (p.vec16 && m0 + BM <= p.M && n0 + BN <= p.N)
+    store_tile_staged<OUT_DT, BIAS_DT, FN, FM, WAVE_BYTES, RES>(acc, p, m0, n0, wn * 32 * FN, wm * 32 * FM, sw_l, b_l,
+                                                                sx_l, hf, l32, lane, smem + w * WAVE_BYTES, g_l);
+  else
+    store_tile<OUT_DT, BIAS_DT, FN, FM, RES>(acc, p, m0, n0, wn * 32 * FN, wm * 32 * FM, BM, BN, sw_l, b_l, sx_l, hf,
+                                             l32, g_l);
 }
-
-#undef DC_WAIT_VMCNT
-#undef DC_WAIT_VMCNT_LGKM0
 
 // Rescale pass over an int32 accumulator (dc_rescale), or over the sum of
 // nsplit split-K partials split_stride apart (exact in int32): one thread
@@ -955,46 +902,54 @@ __global__ void __launch_bounds__(256) rescale_vec_kernel(const int32_t* __restr
   }
 }
 
+// Sets a kernel's dynamic LDS limit, once per instantiation and device
+// (`done`: its flags); threads that race on a first call each set it (the call
+// is idempotent).
+static int reserve_lds(const void* fn, int bytes, std::atomic<bool> (&done)[64], const char* what) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (done[dev].load(std::memory_order_acquire)) return DC_OK;
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) {
+    set_error("%s: cannot reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+    return DC_EHIP;
+  }
+  done[dev].store(true, std::memory_order_release);
+  return DC_OK;
+}
+
 template <class T, int OUT_DT, int BIAS_DT>
 static int launch_gemm(GemmArgs p, hipStream_t st) {
   p.tiles_n = (p.N + T::BN - 1) / T::BN;
   p.tiles_m = (p.M + T::BM - 1) / T::BM;
   const int64_t tiles = (int64_t)p.tiles_n * p.tiles_m;
   if (tiles > 0x7fffffff) return fail(DC_EINVAL, "dc_w8a8_gemm: problem too large");
-  // the LDS attribute, set once per instantiation and device; threads that
-  // race on a first call each set it (the call is idempotent)
   static std::atomic<bool> attr_set[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (!attr_set[dev].load(std::memory_order_acquire)) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&w8a8_gemm_kernel<T, OUT_DT, BIAS_DT>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
-    if (e != hipSuccess) {
-      set_error("w8a8_gemm_kernel: cannot reserve %d bytes of LDS: %s", T::LDS, hipGetErrorString(e));
-      return DC_EHIP;
-    }
-    attr_set[dev].store(true, std::memory_order_release);
-  }
+  if (int e = reserve_lds(reinterpret_cast<const void*>(&w8a8_gemm_kernel<T, OUT_DT, BIAS_DT>), T::LDS, attr_set,
+                          "w8a8_gemm_kernel"))
+    return e;
   const unsigned ks = p.ksplit > 1 ? (unsigned)p.ksplit : 1u;
   hipLaunchKernelGGL((w8a8_gemm_kernel<T, OUT_DT, BIAS_DT>), dim3((unsigned)tiles, ks), dim3(T::NT), T::LDS, st, p);
   return launch_status("w8a8_gemm_kernel");
 }
 
-template <int OUT_DT, int BIAS_DT>
-static int launch_gemm_dma(GemmArgs p, hipStream_t st) {
-  p.tiles_n = (p.N + 255) / 256;
-  p.tiles_m = (p.M + 255) / 256;
-  const int64_t tiles = (int64_t)p.tiles_n * p.tiles_m;
-  if (tiles > 0x7fffffff) return fail(DC_EINVAL, "dc_w8a8_gemm: problem too large");
-  hipLaunchKernelGGL((w8a8_gemm_dma_kernel<OUT_DT, BIAS_DT>), dim3((unsigned)tiles), dim3(256), 0, st, p, GroupArgs{});
-  return launch_status("w8a8_gemm_dma_kernel");
-}
-
-// Grouped launch: g.first[g.ngroup] tiles in all (p holds N, K, tiles_n).
-template <int OUT_DT, int BIAS_DT, bool RES = false>
-static int launch_gemm_dma_group(GemmArgs p, const GroupArgs& g, hipStream_t st) {
-  hipLaunchKernelGGL((w8a8_gemm_dma_kernel<OUT_DT, BIAS_DT, RES>), dim3((unsigned)g.first[g.ngroup]), dim3(256), 0, st,
-                     p, g);
+// One problem (g.ngroup == 0: tiles from p) or a grouped launch
+// (g.first[g.ngroup] tiles in all; p holds N, K, tiles_n).
+template <class T, int OUT_DT, int BIAS_DT, bool RES = false>
+static int launch_gemm_dma(GemmArgs p, const GroupArgs& g, hipStream_t st) {
+  int64_t tiles = g.ngroup ? g.first[g.ngroup] : 0;
+  if (!g.ngroup) {
+    p.tiles_n = (p.N + T::BN - 1) / T::BN;
+    p.tiles_m = (p.M + T::BM - 1) / T::BM;
+    tiles = (int64_t)p.tiles_n * p.tiles_m;
+    if (tiles > 0x7fffffff) return fail(DC_EINVAL, "dc_w8a8_gemm: problem too large");
+  }
+  static std::atomic<bool> attr_set[64];
+  if (int e = reserve_lds(reinterpret_cast<const void*>(&w8a8_gemm_dma_kernel<T, OUT_DT, BIAS_DT, RES>),
+                          T::lds_bytes(RES), attr_set, "w8a8_gemm_dma_kernel"))
+    return e;
+  hipLaunchKernelGGL((w8a8_gemm_dma_kernel<T, OUT_DT, BIAS_DT, RES>), dim3((unsigned)tiles), dim3(T::NT),
+                     T::lds_bytes(RES), st, p, g);
   return launch_status("w8a8_gemm_dma_kernel");
 }
 
@@ -1016,7 +971,7 @@ static int device_cus() {
 // problem takes, that hold useful work (the output area M x N over all the
 // slot-tiles of those rounds, so a tile's padding past M or N counts as
 // waste), weighted by each shape's per-tile efficiency (measured): 256 x 256
-// (the DMA-fed 4-wave kernel when K % 256 == 0, else 8 waves; 1 per CU),
+// (class DMA_256x256 when K % 256 == 0; 1 per CU),
 // 192 (n) x 256 (m) on 8 waves (1 per CU, wave tiles 96 x 64), 128 x 128 on
 // 4 waves (2 per CU). A 4096 x 9216 problem, say, is 576 tiles of
 // 256 x 256 (2.25 rounds on 256 CUs) but exactly 768 of 192 x 256. The
@@ -1034,7 +989,8 @@ static int device_cus() {
 // 8192 x 640 -> 640). Measured: FLUX's 512-row text MLP up 33.2 -> 30.5 us
 // and qkv 31.6 -> 27.8 us; the choice is unchanged on the other SD1.5 /
 // SDXL / FLUX shapes.
-// Kernel plan for a problem: DC_GEMM_PLAN_* (the choice pick_tile launches).
+// Tile class of a problem: DC_GEMM_PLAN_* (dc_w8a8_gemm_plan; pick_tile runs it on
+// the register-staged kernel where pick_dma has no tile).
 static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
   struct Cand { int bn, bm, per_cu; float eff; };
   const int cus = device_cus();
@@ -1053,22 +1009,79 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
     if (score > best_score) best = i, best_score = score;
   }
   if (best == 0) {
-    // 256 x 256 tiles: the DMA-fed kernel when its shape conditions hold
-    if (K % (4 * DBK) == 0 && 256 * lda < (int64_t(1) << 31) && 256 * ldw < (int64_t(1) << 31))
+    if (K % 256 == 0 && 256 * lda < (int64_t(1) << 31) && 256 * ldw < (int64_t(1) << 31))
       return DC_GEMM_PLAN_DMA_256x256;
     return DC_GEMM_PLAN_256x256;
   }
   return best == 1 ? DC_GEMM_PLAN_192x256 : best == 2 ? DC_GEMM_PLAN_128x128 : DC_GEMM_PLAN_192x128;
 }
 
+// Tile of the DMA-fed kernel for a problem, or none (the register-staged
+// kernel of plan_tile's shape runs it). By how many 128 x 128 tiles (t128) the
+// problem holds, on 256 CUs; graph time per call over rotating operands, fp16
+// out, against the register-staged kernel (or the 64-byte-stage 256 x 256
+// one) that ran the size before:
+//   t128 <= CUs / 2: smaller tiles spread the work (and the weight bytes, what
+//     bounds these) over more CUs. 64 x 64 while 64 x 128 tiles would fill
+//     under half the CUs: 154 x 2048 -> 2560 14.4 -> 6.8 us (64 x 128: 8.0;
+//     128 x 128: 9.8); else 64 x 128: 512 x 3072 -> 3072 21.5 -> 11.7 (64 x 64:
+//     12.2), 512 x 12288 -> 3072 38.8 -> 33.5 (36.8; 128 x 128: 40).
+//   t128 <= CUs: one 8-wave 128 x 128 tile per CU, two waves per SIMD and 3
+//     stages to hide the loads no other workgroup hides: 2048 x 1280 -> 1280
+//     11.3 -> 8.6 (4 waves, two stages: 10.4), 2048 x 5120 -> 1280 30.3 -> 21.2
+//     (29.2).
+//   t128 <= 2 CUs: two 4-wave 128 x 128 workgroups per CU, one's epilogue
+//     under the other's products: 2048 x 1280 -> 3840 17.4 -> 14.2 (256 x 256:
+//     18.9), 8192 x 2560 -> 640 26.8 -> 19.8 (29.7).
+//   above: the least time by a fit of the measured times, a fixed part and a
+//     part per round of the device's slots, linear in K. A last round of
+//     128 x 128 tiles that puts one on each CU takes 0.65 of a full one; the
+//     large tiles' fixed part is a prologue and an epilogue with no other
+//     workgroup to run beside. 4096 x 3072 -> 9216: 192 x 256 123.2 -> 119.7
+//     (256 x 256: 130.9, 128 x 128: 135.1); 4608 x 3072 -> 21504: 256 x 256
+//     306.8 -> 280.8 (128 x 128: 315.4); 8192 x 640 -> 5120: 128 x 128 49.2 ->
+//     42.6 (256 x 256: 43.2).
+// K = 64 (mod 128): 64-byte stages at 128 x 128, 3 workgroups per CU; 8192 x
+// 320 -> 1280 with float32 out 18.4 -> 12.7 us. Only below K = 1024: deeper
+// ones would want the larger tiles of the register-staged kernel.
+enum DmaPick { DMA_NONE, DMA_256x256, DMA_192x256, DMA_128x128, DMA_128x128D, DMA_64x128, DMA_64x64, DMA_128x128K };
+static DmaPick pick_dma(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
+  if (K % 64 || 256 * lda >= (int64_t(1) << 31) || 256 * ldw >= (int64_t(1) << 31)) return DMA_NONE;
+  if (K % 128) return K < 1024 ? DMA_128x128K : DMA_NONE;
+  const int64_t cus = device_cus();
+  const auto tiles = [&](int bn, int bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+  const int64_t t128 = tiles(128, 128);
+  if (t128 <= cus / 2) return tiles(64, 128) < cus / 2 ? DMA_64x64 : DMA_64x128;
+  if (t128 <= cus) return DMA_128x128D;
+  if (t128 <= 2 * cus) return DMA_128x128;
+  const double k = (double)K;
+  const auto rounds = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
+  const int64_t full = t128 / (2 * cus), rest = t128 % (2 * cus);
+  const double c128 = 1.5 + ((double)full + (rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0)) * (3.4 + 0.0080 * k);
+  const double c192 = 5.0 + rounds(tiles(192, 256)) * (2.5 + 0.0112 * k);
+  const double c256 = 6.4 + rounds(tiles(256, 256)) * (4.0 + 0.0135 * k);
+  if (c128 <= c192 && c128 <= c256) return DMA_128x128;
+  return c192 < c256 ? DMA_192x256 : DMA_256x256;
+}
+
 template <int OUT_DT, int BIAS_DT>
 static int pick_tile(GemmArgs p, hipStream_t st) {
+  const GroupArgs one{};
+  switch (pick_dma(p.M, p.N, p.K, p.lda, p.ldw)) {
+    case DMA_256x256: return launch_gemm_dma<Dma256x256, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_192x256: return launch_gemm_dma<Dma192x256, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_128x128: return launch_gemm_dma<Dma128x128, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_128x128D: return launch_gemm_dma<Dma128x128d, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_64x128: return launch_gemm_dma<Dma64x128, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_64x64: return launch_gemm_dma<Dma64x64, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_128x128K: return launch_gemm_dma<Dma128x128k, OUT_DT, BIAS_DT>(p, one, st);
+    case DMA_NONE: break;
+  }
   switch (plan_tile(p.M, p.N, p.K, p.lda, p.ldw)) {
-    case DC_GEMM_PLAN_DMA_256x256: return launch_gemm_dma<OUT_DT, BIAS_DT>(p, st);
-    case DC_GEMM_PLAN_256x256: return launch_gemm<Tile<2, 4, 4, 2, 1>, OUT_DT, BIAS_DT>(p, st);
     case DC_GEMM_PLAN_192x256: return launch_gemm<Tile<2, 4, 3, 2, 1>, OUT_DT, BIAS_DT>(p, st);
     case DC_GEMM_PLAN_192x128: return launch_gemm<Tile<2, 2, 3, 2, 1>, OUT_DT, BIAS_DT>(p, st);
-    default: return launch_gemm<Tile<2, 2, 2, 2, 1>, OUT_DT, BIAS_DT>(p, st);
+    case DC_GEMM_PLAN_128x128: return launch_gemm<Tile<2, 2, 2, 2, 1>, OUT_DT, BIAS_DT>(p, st);
+    default: return launch_gemm<Tile<2, 4, 4, 2, 1>, OUT_DT, BIAS_DT>(p, st);
   }
 }
 
@@ -1191,7 +1204,8 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
     return fail(DC_EINVAL, "dc_w8a8_gemm: bad bias_dtype");
   // split-K into the workspace (int32 partials), then the epilogue over their sum
   int kslice = 0;
-  const int ks = (out_dtype != DC_I32 && workspace) ? splitk_plan(M, N, K, lda, ldw, &kslice) : 1;
+  const int ks = (out_dtype != DC_I32 && workspace && pick_dma(M, N, K, lda, ldw) == DMA_NONE)
+                     ? splitk_plan(M, N, K, lda, ldw, &kslice) : 1;
   if (ks > 1 && ws_bytes >= (size_t)ks * (size_t)M * (size_t)N * 4 && aligned16(workspace)) {
     GemmArgs q = p;
     q.sx = nullptr; q.sw = nullptr; q.bias = nullptr;
@@ -1224,10 +1238,10 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
 template <int OUT_DT, bool RES = false>
 static int group_bias(GemmArgs p, const GroupArgs& g, int bias_dtype, hipStream_t st) {
   switch (bias_dtype) {
-    case DC_NONE: return launch_gemm_dma_group<OUT_DT, DC_NONE, RES>(p, g, st);
-    case DC_F16: return launch_gemm_dma_group<OUT_DT, DC_F16, RES>(p, g, st);
-    case DC_BF16: return launch_gemm_dma_group<OUT_DT, DC_BF16, RES>(p, g, st);
-    default: return launch_gemm_dma_group<OUT_DT, DC_F32, RES>(p, g, st);
+    case DC_NONE: return launch_gemm_dma<Dma256x256, OUT_DT, DC_NONE, RES>(p, g, st);
+    case DC_F16: return launch_gemm_dma<Dma256x256, OUT_DT, DC_F16, RES>(p, g, st);
+    case DC_BF16: return launch_gemm_dma<Dma256x256, OUT_DT, DC_BF16, RES>(p, g, st);
+    default: return launch_gemm_dma<Dma256x256, OUT_DT, DC_F32, RES>(p, g, st);
   }
 }
 
@@ -1252,7 +1266,7 @@ extern "C" int dc_w8a8_gemm_group_plan(const int64_t* Ms, int count, int64_t N, 
     total += t;
     largest = t > largest ? t : largest;
   }
-  if (K % (4 * DBK) || live < 2) return 0;
+  if (K % 256 || live < 2) return 0;
   const int64_t cus = device_cus();
   return (total + cus - 1) / cus <= (largest + cus - 1) / cus ? 1 : 0;
 }
@@ -1271,7 +1285,7 @@ static int group_setup(const char* who, const dc_gemm_problem* problems, const d
   if (count < 1 || count > DC_GEMM_MAX_GROUP) return group_fail(DC_EINVAL, who, "count must be 1 .. DC_GEMM_MAX_GROUP");
   if (N <= 0 || K <= 0) return group_fail(DC_EINVAL, who, "N and K must be positive");
   if (N > 0x7fffffff || K > 0x7fffffff) return group_fail(DC_EINVAL, who, "size too large");
-  if (K % (4 * DBK)) return group_fail(DC_EUNSUPPORTED, who, "needs K % 256 == 0");
+  if (K % 256) return group_fail(DC_EUNSUPPORTED, who, "needs K % 256 == 0");
   if (out_dtype != DC_I32 && out_dtype != DC_F16 && out_dtype != DC_BF16 && out_dtype != DC_F32)
     return group_fail(DC_EINVAL, who, "bad out_dtype");
   if (bias_dtype != DC_NONE && bias_dtype != DC_F16 && bias_dtype != DC_BF16 && bias_dtype != DC_F32)
@@ -1337,7 +1351,7 @@ extern "C" int dc_w8a8_gemm_grouped(const dc_gemm_problem* problems, int count, 
   if (g.ngroup == 0) return DC_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (out_dtype) {
-    case DC_I32: return launch_gemm_dma_group<DC_I32, DC_NONE>(p, g, st);
+    case DC_I32: return launch_gemm_dma<Dma256x256, DC_I32, DC_NONE>(p, g, st);
     case DC_F16: return group_bias<DC_F16>(p, g, bias_dtype, st);
     case DC_BF16: return group_bias<DC_BF16>(p, g, bias_dtype, st);
     default: return group_bias<DC_F32>(p, g, bias_dtype, st);

@@ -145,8 +145,8 @@ int dc_qk_norm_rope(int dtype, int64_t B, int64_t L, int64_t H, int64_t D, int f
  *   and int_mm + rescale (_int8.py:313-323), rounding bit for bit like them.
  * Needs K % 16 == 0, lda % 16 == 0, ldw % 16 == 0 and 16-byte aligned a, w.
  * workspace / ws_bytes (may be NULL / 0): scratch for split-K on problems
- * whose tiles would leave most of the device idle (small M, long K; see
- * dc_w8a8_gemm_workspace_bytes). The k range is split over workgroups that
+ * whose tiles would leave most of the device idle (small M, long K, no small
+ * DMA-fed tile; see dc_w8a8_gemm_workspace_bytes). The k range is split over workgroups that
  * write int32 partial sums there, and an epilogue pass adds them (exact) and
  * applies the same rescale, bias and cast: results are bit-identical to the
  * unsplit call. Without enough workspace the call runs unsplit.
@@ -157,24 +157,27 @@ int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, con
                  void* stream);
 
 /*
- * Workspace bytes dc_w8a8_gemm uses for split-K on this problem on the
+ * Workspace bytes dc_w8a8_gemm may use for split-K on this problem on the
  * current device (0: it runs unsplit). No counterpart in the reference, whose
  * GEMMs are torch._int_mm and one CUTLASS kernel (_int8.py:200-276).
  */
 size_t dc_w8a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw);
 
 /*
- * Which GEMM kernel dc_w8a8_gemm runs for a problem on the current device:
- * one of the DC_GEMM_PLAN_* codes, or -1 for a shape it rejects. Tiles are
- * chosen by how full the last round of workgroups keeps the device. No
+ * Tile class of a dc_w8a8_gemm problem on the current device: one of the
+ * DC_GEMM_PLAN_* codes, or -1 for a shape it rejects. Classes are chosen by how
+ * full the last round of workgroups keeps the device. K that is not a multiple
+ * of 64 runs exactly that tile; other K run on the DMA-fed kernel, whose own
+ * rule may take another tile of it. A problem of class DMA_256x256 is one that
+ * dc_w8a8_gemm_grouped(_gated) takes without losing to dc_w8a8_gemm. No
  * counterpart in the reference (its GEMMs come from torch._int_mm and one
- * CUTLASS configuration, _int8.py:200-276); for profiling and tests.
+ * CUTLASS configuration, _int8.py:200-276); for profiling, dispatch and tests.
  */
 enum {
   DC_GEMM_PLAN_256x256 = 0,      /* 8 waves, 128 x 64 wave tiles, register-staged loads */
   DC_GEMM_PLAN_192x256 = 1,      /* 8 waves, 96 x 64 wave tiles */
   DC_GEMM_PLAN_128x128 = 2,      /* 4 waves, 64 x 64 wave tiles, 2 workgroups per CU */
-  DC_GEMM_PLAN_DMA_256x256 = 3,  /* 4 waves, 128 x 128 wave tiles, loads straight into LDS */
+  DC_GEMM_PLAN_DMA_256x256 = 3,  /* 8 waves, 64 x 128 wave tiles, loads straight into LDS */
   DC_GEMM_PLAN_192x128 = 4       /* 192 (n) x 128 (m) on 4 waves, 96 x 64 wave tiles, 1 workgroup per CU */
 };
 int dc_w8a8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw);

@@ -470,3 +470,40 @@ def test_multi_round_grouped_gemm_bit_exact(gpu, ms, n, k, dtype, bias_dtype):
     for (q, w, sx, sw, b), out in zip(items, outs):
         assert torch.equal(out, _int32_then_rescale(q, w, sx, sw, b, dtype))
     assert all(torch.equal(a, c) for a, c in zip(_int8._gemm_grouped(items, dtype), outs))
+
+
+# The DMA-fed kernel's tiles (64 x 64, 64 x 128, 128 x 128 one and two per CU,
+# 192 x 256, 256 x 256; 128 x 128 with 64-byte stages for K = 64 mod 128) at
+# whole and ragged edges, with fewer k stages than the ring holds, as many, and
+# one or two more; the last ones leave K % 64 or its depth to the
+# register-staged kernel.
+DMA_EDGES = [(1, 8, 128), (64, 64, 256), (65, 130, 384), (154, 2560, 512), (129, 513, 128), (512, 3071, 640),
+             (500, 3072, 1280), (1000, 2048, 256), (1025, 2049, 384), (2048, 1281, 512), (2047, 3840, 128),
+             (2000, 3840, 640), (4096, 3072, 1024), (4095, 3001, 384), (2560, 16384, 256), (2500, 16380, 384),
+             (7904, 1920, 640), (1, 4, 64), (130, 260, 192), (8192, 1280, 320), (3000, 1284, 576), (100, 100, 960),
+             (257, 300, 1088), (300, 200, 48)]
+
+
+@pytest.mark.parametrize("mnk", DMA_EDGES)
+def test_dma_tiles_bit_exact(gpu, mnk):
+    """Every tile and edge against the vendor's int32 product and the rescale
+    expression in torch ops, from operands that are slices of wider rows
+    (strides above K) into an output of every type."""
+    m, n, k = mnk
+    g = torch.Generator(device=gpu).manual_seed(m * 7 + n + k)
+    wide = k + 32
+    q = torch.randint(-128, 128, (m, wide), generator=g, device=gpu, dtype=torch.int8)[:, 16:16 + k]
+    w = torch.randint(-128, 128, (n, wide), generator=g, device=gpu, dtype=torch.int8)[:, 16:16 + k]
+    sx, sw = (torch.rand(i, generator=g, device=gpu) * 1e-3 for i in (m, n))
+    bias = torch.randn(n, generator=g, device=gpu)
+    # the vendor product needs M > 16 and sizes that are multiples of 8
+    mp, np_ = (max(m, 32) + 7) // 8 * 8, (n + 7) // 8 * 8
+    qp, wp = torch.zeros(mp, k, device=gpu, dtype=torch.int8), torch.zeros(np_, k, device=gpu, dtype=torch.int8)
+    qp[:m], wp[:n] = q, w
+    acc = torch._int_mm(qp, wp.t())[:m, :n]
+    assert torch.equal(_int8._gemm(q, w, None, None, None, torch.int32), acc)
+    for dtype, b in ((torch.bfloat16, bias.bfloat16()), (torch.float16, None), (torch.float32, bias)):
+        y = (acc.float() * (sx.unsqueeze(-1) * sw)).to(dtype)
+        if b is not None:
+            y = y + b.to(dtype)
+        assert torch.equal(_int8._gemm(q, w, sx, sw, b, dtype), y), dtype
