@@ -468,18 +468,20 @@ __device__ __forceinline__ void store_tile_staged(const v16i (&acc)[FN][FM], con
   }
 }
 
+// Split-K: this workgroup's slice of k and its partial sums.
+__device__ __forceinline__ void split_slice(GemmArgs& p) {
+  if (p.ksplit <= 1) return;
+  const int k0 = (int)blockIdx.y * p.kslice;
+  p.a += k0;
+  p.w += k0;
+  p.K = min(p.kslice, p.K - k0);
+  p.out = static_cast<int32_t*>(p.out) + (int64_t)blockIdx.y * p.split_stride;
+}
+
 template <class T, int OUT_DT, int BIAS_DT>
 __global__ void __launch_bounds__(T::NT, 1) w8a8_gemm_kernel(GemmArgs p) {
   constexpr int FN = T::FN, FM = T::FM, NT = T::NT;
-  if constexpr (OUT_DT == DC_I32) {
-    if (p.ksplit > 1) {
-      const int k0 = (int)blockIdx.y * p.kslice;
-      p.a += k0;
-      p.w += k0;
-      p.K = min(p.kslice, p.K - k0);
-      p.out = static_cast<int32_t*>(p.out) + (int64_t)blockIdx.y * p.split_stride;
-    }
-  }
+  if constexpr (OUT_DT == DC_I32) split_slice(p);
   constexpr int BN = T::BN, BM = T::BM;
   constexpr int CPR = BK / 16;                    // 16-byte chunks per row
   constexpr int NWL = BN * CPR / NT, NAL = BM * CPR / NT;
@@ -710,6 +712,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) w8a8_gemm_dma_kernel(GemmArgs p
   constexpr int FN = T::FN, FM = T::FM, BN = T::BN, BM = T::BM, S = T::S, KB = T::KB, L = T::LW + T::LA;
   constexpr int NKS = KB / 32;   // MFMA k-steps per stage
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  if constexpr (OUT_DT == DC_I32) split_slice(p);
 
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int l32 = lane & 31, hf = lane >> 5;
@@ -809,7 +812,13 @@ __global__ void __launch_bounds__(T::NT, T::OCC) w8a8_gemm_dma_kernel(GemmArgs p
 #pragma unroll
     for (int ks = 0; ks < NKS - 1; ++ks) {
       frags((ks + 1) & 1, slot, ks + 1);
+      // the one-block waves, two or three workgroups per CU: a wave that has its
+      // fragments goes ahead of the others' DMA set-up (512 x 12288 -> 3072
+      // 33.4 -> 30.9 us, 154 x 2048 -> 2560 6.8 -> 6.2; level on 128 x 128
+      // tiles, 2.5% slower on 256 x 256 ones)
+      if constexpr (FN * FM == 1) __builtin_amdgcn_s_setprio(1);
       mfmas(ks & 1);
+      if constexpr (FN * FM == 1) __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
     }
     const int next = slot == S - 1 ? 0 : slot + 1;
@@ -817,8 +826,17 @@ __global__ void __launch_bounds__(T::NT, T::OCC) w8a8_gemm_dma_kernel(GemmArgs p
     else wait_left(nk - 2 - kt);
     wait_lgkmcnt0();
     sync();
-    if constexpr (MORE) issue(kt + S, slot);
-    frags(0, next, 0);
+    // the large tiles' 7 or 8 DMAs per wave go after the fragment reads, whose
+    // latency then runs under their issue (4096 x 12288 -> 3072 141.8 -> 137.5
+    // us, 4096 x 3072 -> 9216 120.1 -> 116.8; level elsewhere)
+    if constexpr (FN * FM >= 6) {
+      frags(0, next, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (MORE) issue(kt + S, slot);
+    } else {
+      if constexpr (MORE) issue(kt + S, slot);
+      frags(0, next, 0);
+    }
     mfmas(1);
     __builtin_amdgcn_sched_barrier(0);
     slot = next;
@@ -948,7 +966,8 @@ static int launch_gemm_dma(GemmArgs p, const GroupArgs& g, hipStream_t st) {
   if (int e = reserve_lds(reinterpret_cast<const void*>(&w8a8_gemm_dma_kernel<T, OUT_DT, BIAS_DT, RES>),
                           T::lds_bytes(RES), attr_set, "w8a8_gemm_dma_kernel"))
     return e;
-  hipLaunchKernelGGL((w8a8_gemm_dma_kernel<T, OUT_DT, BIAS_DT, RES>), dim3((unsigned)tiles), dim3(T::NT),
+  const unsigned ks = p.ksplit > 1 ? (unsigned)p.ksplit : 1u;
+  hipLaunchKernelGGL((w8a8_gemm_dma_kernel<T, OUT_DT, BIAS_DT, RES>), dim3((unsigned)tiles, ks), dim3(T::NT),
                      T::lds_bytes(RES), st, p, g);
   return launch_status("w8a8_gemm_dma_kernel");
 }
@@ -1023,9 +1042,9 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
 // one) that ran the size before:
 //   t128 <= CUs / 2: smaller tiles spread the work (and the weight bytes, what
 //     bounds these) over more CUs. 64 x 64 while 64 x 128 tiles would fill
-//     under half the CUs: 154 x 2048 -> 2560 14.4 -> 6.8 us (64 x 128: 8.0;
-//     128 x 128: 9.8); else 64 x 128: 512 x 3072 -> 3072 21.5 -> 11.7 (64 x 64:
-//     12.2), 512 x 12288 -> 3072 38.8 -> 33.5 (36.8; 128 x 128: 40).
+//     under half the CUs: 154 x 2048 -> 2560 14.4 -> 6.2 us (64 x 128: 7.2;
+//     128 x 128: 9.8); else 64 x 128: 512 x 3072 -> 3072 21.5 -> 10.7 (64 x 64:
+//     11.9), 512 x 12288 -> 3072 38.8 -> 30.9 (36.5; 128 x 128: 40).
 //   t128 <= CUs: one 8-wave 128 x 128 tile per CU, two waves per SIMD and 3
 //     stages to hide the loads no other workgroup hides: 2048 x 1280 -> 1280
 //     11.3 -> 8.6 (4 waves, two stages: 10.4), 2048 x 5120 -> 1280 30.3 -> 21.2
@@ -1154,6 +1173,19 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw
   return (int)((K + slice - 1) / slice);
 }
 
+// The same for a problem the DMA-fed kernel takes: its small tiles leave split-K
+// only the deepest products on the fewest rows (the partials and the second
+// launch cost about 4 us): 4 slices of 64 x 64 tiles from K = 8192 when those
+// tiles cover at most 3/4 of the CUs. 64 x 12288 -> 3072 23.8 -> 13.2 us,
+// 256 x 12288 -> 3072 25.2 -> 22.7; at 512 rows (64 x 128 tiles) 31.6 -> 35.5,
+// 154 x 2048 -> 1280 6.6 -> 8.5. K % 512 == 0 keeps the slices whole stages.
+static int dma_splits(int64_t M, int64_t N, int64_t K, int* kslice) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (K < 8192 || K % 512 || 4 * tiles > 3 * (int64_t)device_cus()) return 1;
+  *kslice = (int)(K / 4);
+  return 4;
+}
+
 }  // namespace dc
 
 using namespace dc;
@@ -1204,8 +1236,12 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
     return fail(DC_EINVAL, "dc_w8a8_gemm: bad bias_dtype");
   // split-K into the workspace (int32 partials), then the epilogue over their sum
   int kslice = 0;
-  const int ks = (out_dtype != DC_I32 && workspace && pick_dma(M, N, K, lda, ldw) == DMA_NONE)
-                     ? splitk_plan(M, N, K, lda, ldw, &kslice) : 1;
+  int ks = (out_dtype != DC_I32 && workspace) ? splitk_plan(M, N, K, lda, ldw, &kslice) : 1;
+  const bool dma = ks > 1 && pick_dma(M, N, K, lda, ldw) != DMA_NONE;
+  if (dma) {   // the caller's workspace holds splitk_plan's slices
+    const int n = dma_splits(M, N, K, &kslice);
+    ks = ks >= n ? n : 1;
+  }
   if (ks > 1 && ws_bytes >= (size_t)ks * (size_t)M * (size_t)N * 4 && aligned16(workspace)) {
     GemmArgs q = p;
     q.sx = nullptr; q.sw = nullptr; q.bias = nullptr;
@@ -1216,7 +1252,9 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
     q.ksplit = ks;
     q.kslice = kslice;
     q.split_stride = M * N;
-    if (int e = launch_gemm<Tile<2, 2, 2, 2, 1>, DC_I32, DC_NONE>(q, st)) return e;
+    if (int e = dma ? launch_gemm_dma<Dma64x64, DC_I32, DC_NONE>(q, GroupArgs{}, st)
+                    : launch_gemm<Tile<2, 2, 2, 2, 1>, DC_I32, DC_NONE>(q, st))
+      return e;
     const int32_t* acc = static_cast<const int32_t*>(workspace);
     switch (out_dtype) {
       case DC_F16: return rescale_bias<DC_F16>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, ks, M * N);

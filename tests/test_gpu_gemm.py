@@ -507,3 +507,15 @@ def test_dma_tiles_bit_exact(gpu, mnk):
         if b is not None:
             y = y + b.to(dtype)
         assert torch.equal(_int8._gemm(q, w, sx, sw, b, dtype), y), dtype
+
+
+@pytest.mark.parametrize("mnk", [(64, 3072, 12288), (100, 3069, 8192), (1, 16, 8704), (256, 3072, 15360)])
+def test_dma_split_k_bit_exact(gpu, mnk):
+    """Few rows over a deep K: four k slices of the DMA-fed kernel's smallest
+    tile (the workspace the library asks for) equal the unsplit call."""
+    m, n, k = mnk
+    q, w, sx, sw = (t.to(gpu) for t in _qw(m, n, k, 17))
+    bias = torch.randn(n, device=gpu).bfloat16()
+    assert _lib.require().dc_w8a8_gemm_workspace_bytes(m, n, k, k, k) >= 4 * m * n * 4
+    for dtype, b in ((torch.bfloat16, bias), (torch.float32, None)):
+        assert torch.equal(_int8._gemm(q, w, sx, sw, b, dtype), _gemm_unsplit(q, w, sx, sw, b, dtype))
