@@ -29,6 +29,9 @@ _SIGS = {
     "dc_abi_version": (_I, []),
     "dc_quantize_rows": (_I, [_P, _I, _I64, _I64, _I64, _I, _P, _I64, _P, _P]),
     "dc_w8a8_gemm": (_I, [_P, _I64, _P, _I64, _P, _P, _P, _I, _P, _I, _I64, _I64, _I64, _I64, _P, ctypes.c_size_t, _P]),
+    "dc_w8a8_linear": (_I, [_P, _I, _I64, _I64, _I64, _I, _P, _I64, _P, _P, _I, _P, _I, _I64, _I64, _P,
+                            ctypes.c_size_t, _P]),
+    "dc_w8a8_linear_scratch_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _I64]),
     "dc_w8a8_gemm_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64]),
     "dc_w8a8_gemm_plan": (_I, [_I64, _I64, _I64, _I64, _I64]),
     "dc_w8a8_gemm_grouped": (_I, [_P, _I, _I64, _I64, _I, _I, _P]),
@@ -121,6 +124,10 @@ def check(rc: int, what: str) -> None:
 # torch's raw current-stream query (the handle only, no Stream object: about
 # 0.1 us against 3 us per call); the public API where it is missing
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# the current device's index the same way (0.1 us against 0.5); torch's own
+# function initializes the runtime first, which a GPU tensor already has
+_raw_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_HERE = contextlib.nullcontext()
 
 
 def stream_ptr(device: torch.device) -> int:
@@ -136,8 +143,8 @@ def device_ctx(device: torch.device):
     device that is not a GPU raises: the kernels take device pointers only."""
     if device.type != "cuda":
         raise RuntimeError(f"diffucore_amd: the HIP kernels take GPU tensors (got a {device} tensor)")
-    if device.index is None or device.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
+    if device.index is None or device.index == _raw_device():
+        return _HERE
     return torch.cuda.device(device)
 
 

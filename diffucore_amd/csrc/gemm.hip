@@ -1271,6 +1271,38 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
   }
 }
 
+// ---------------------------------------------------------------- whole layer
+
+static size_t pad256(size_t n) { return (n + 255) / 256 * 256; }
+
+// scratch: codes [M, K], row scales [M], then the GEMM's split-K workspace
+extern "C" size_t dc_w8a8_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t ldw) {
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+  return pad256((size_t)M * (size_t)K) + pad256((size_t)M * 4) + dc_w8a8_gemm_workspace_bytes(M, N, K, K, ldw);
+}
+
+extern "C" int dc_w8a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int group,
+                              const int8_t* w, int64_t ldw, const float* sw, const void* bias, int bias_dtype,
+                              void* out, int out_dtype, int64_t ldo, int64_t N, void* scratch, size_t scratch_bytes,
+                              void* stream) {
+  clear_error();
+  if (M < 0 || N < 0 || K <= 0) return fail(DC_EINVAL, "dc_w8a8_linear: bad M/N/K");
+  if (M == 0 || N == 0) return DC_OK;
+  if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return fail(DC_EINVAL, "dc_w8a8_linear: size too large");
+  if (K % 16) return fail(DC_EUNSUPPORTED, "dc_w8a8_linear: needs K % 16 == 0");
+  if (out_dtype != DC_F16 && out_dtype != DC_BF16 && out_dtype != DC_F32)
+    return fail(DC_EINVAL, "dc_w8a8_linear: out_dtype must be DC_F16, DC_BF16 or DC_F32");
+  if (!scratch || !aligned16(scratch) || scratch_bytes < dc_w8a8_linear_scratch_bytes(M, N, K, ldw))
+    return fail(DC_EWORKSPACE, "dc_w8a8_linear: scratch too small or not 16-byte aligned");
+  int8_t* q = static_cast<int8_t*>(scratch);
+  float* sx = reinterpret_cast<float*>(q + pad256((size_t)M * (size_t)K));
+  uint8_t* ws = reinterpret_cast<uint8_t*>(sx) + pad256((size_t)M * 4);
+  const size_t ws_bytes = scratch_bytes - (size_t)(ws - static_cast<uint8_t*>(scratch));
+  if (int e = dc_quantize_rows(x, x_dtype, M, K, ldx, group, q, K, sx, stream)) return e;
+  return dc_w8a8_gemm(q, K, w, ldw, sx, sw, bias, bias_dtype, out, out_dtype, ldo, M, N, K, ws_bytes ? ws : nullptr,
+                      ws_bytes, stream);
+}
+
 // ---------------------------------------------------------------- grouped launches
 
 template <int OUT_DT, bool RES = false>

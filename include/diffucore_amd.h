@@ -164,6 +164,20 @@ int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, con
 size_t dc_w8a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw);
 
 /*
+ * A whole W8A8 layer in one call: dc_quantize_rows of x, then dc_w8a8_gemm of
+ * the codes, with both calls' rules and results (two launches, three when the
+ * GEMM splits k). The codes, row scales and split-K partials live in `scratch`
+ * (16-byte aligned, at least dc_w8a8_linear_scratch_bytes), whose contents
+ * need not survive the call and need not start at zero. K % 16 == 0.
+ * Replaces Int8Linear.forward (src/diffucore/models/_int8.py:158-167), one
+ * host call per layer instead of one per kernel.
+ */
+int dc_w8a8_linear(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, int group, const int8_t* w,
+                   int64_t ldw, const float* sw, const void* bias, int bias_dtype, void* out, int out_dtype,
+                   int64_t ldo, int64_t N, void* scratch, size_t scratch_bytes, void* stream);
+size_t dc_w8a8_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t ldw);
+
+/*
  * Tile class of a dc_w8a8_gemm problem on the current device: one of the
  * DC_GEMM_PLAN_* codes, or -1 for a shape it rejects. Classes are chosen by how
  * full the last round of workgroups keeps the device. K that is not a multiple

@@ -519,3 +519,56 @@ def test_dma_split_k_bit_exact(gpu, mnk):
     assert _lib.require().dc_w8a8_gemm_workspace_bytes(m, n, k, k, k) >= 4 * m * n * 4
     for dtype, b in ((torch.bfloat16, bias), (torch.float32, None)):
         assert torch.equal(_int8._gemm(q, w, sx, sw, b, dtype), _gemm_unsplit(q, w, sx, sw, b, dtype))
+
+
+@pytest.mark.parametrize("shape,n,group,dtype,bias", [
+    ((154, 2048), 2560, 256, torch.float16, None), ((2, 77, 768), 640, 256, torch.bfloat16, torch.float32),
+    ((1, 320), 4, 0, torch.float32, torch.float32), ((320,), 17, 0, torch.float16, torch.float16),
+    ((64, 12288), 3072, 256, torch.bfloat16, torch.bfloat16), ((3, 0, 256), 64, 256, torch.float16, None),
+    ((33, 48), 100, 0, torch.float16, torch.float16)])
+def test_linear_one_call_equals_two(gpu, shape, n, group, dtype, bias):
+    """Int8Linear.forward (one library call) against quantize_activation and
+    matmul_quantized, on whole and strided inputs and strided weights."""
+    k = shape[-1]
+    torch.manual_seed(n)
+    m = _int8.Int8Linear(k, n, bias=bias is not None, group=group, device=gpu)
+    m.weight.copy_(torch.randint(-127, 128, (n, k), device=gpu))
+    m.scale_bits.copy_((torch.rand(n, device=gpu) * 1e-3).view(torch.int32))
+    if bias is not None:
+        m.bias = nn.Parameter(torch.randn(n, device=gpu).to(bias), requires_grad=False)
+    x = torch.randn(*shape, device=gpu).to(dtype)
+    wide = torch.randn(*shape[:-1], k + 16, device=gpu).to(dtype)
+    odd = torch.randn(*shape[:-1], k + 1, device=gpu).to(dtype)
+    for xi in (x, wide[..., 8:8 + k], odd[..., :k], torch.stack((x, x), -1)[..., 0]):
+        q, s = _int8.quantize_activation(xi.reshape(-1, k), group)
+        want = m.matmul_quantized(q, s, dtype).view(*xi.shape[:-1], n)
+        y = m(xi)
+        assert y.shape == want.shape and y.dtype == dtype and torch.equal(y, want)
+    store = torch.empty(n, k + 64, device=gpu, dtype=torch.int8)
+    store[:, 32:32 + k] = m.weight
+    want = m(x)
+    m.weight = store[:, 32:32 + k]
+    assert torch.equal(m(x), want)
+
+
+def test_linear_one_call_refusals(gpu):
+    """What the two calls refuse, the one call refuses: a width that is not
+    the layer's, a scratch too small, a bias of another type."""
+    m = _int8.Int8Linear(256, 64, group=256, device=gpu)
+    with pytest.raises((RuntimeError, ValueError)):
+        m(torch.randn(4, 512, device=gpu).half())
+    so = _lib.require()
+    x, w = torch.randn(4, 256, device=gpu).half(), torch.zeros(64, 256, device=gpu, dtype=torch.int8)
+    sw, out, scratch = torch.ones(64, device=gpu), torch.empty(4, 64, device=gpu).half(), \
+        torch.empty(4096, device=gpu, dtype=torch.uint8)
+    need = so.dc_w8a8_linear_scratch_bytes(4, 64, 256, 256)
+    args = lambda k, out_dt, nb: (x.data_ptr(), _lib.F16, 4, k, 256, 256, w.data_ptr(), 256, sw.data_ptr(), None,
+                                  _lib.NONE, out.data_ptr(), out_dt, 64, 64, scratch.data_ptr(), nb,
+                                  _lib.stream_ptr(gpu))
+    assert so.dc_w8a8_linear(*args(256, _lib.F16, need)) == 0
+    assert so.dc_w8a8_linear(*args(256, _lib.F16, need - 1)) != 0
+    assert so.dc_w8a8_linear(*args(250, _lib.F16, 4096)) != 0
+    assert so.dc_w8a8_linear(*args(256, _lib.I32, 4096)) != 0
+    m.bias = nn.Parameter(torch.zeros(64, device=gpu, dtype=torch.float64), requires_grad=False)
+    with pytest.raises(TypeError):
+        m(x)
