@@ -19,10 +19,15 @@
 // for all of them, and each lane issues all its loads before any arithmetic.
 // A workgroup of 256 threads takes 256/(D/8) lane groups. q, k and an
 // optional plain copy of v (to gather two
-// streams' v into one buffer for the attention) run in one launch, one
-// contiguous range of workgroups each. The kernel is bound by HBM: 2 bytes
-// read and 2 written per element, the weights and the frequency rows come
-// from cache.
+// streams' v into one buffer for the attention) run in one launch, taking
+// turns 8 workgroups at a time. The kernel is bound by HBM: 2 bytes read and
+// 2 written per element, the weights and the frequency rows come from cache.
+// With one contiguous range of workgroups each for q, k and v instead, the
+// three passes over a stacked [.., 3, H, D] projection each skipped two thirds
+// of every row and read the frequency rows from HBM again: 4096 tokens x 24
+// heads x 128 bf16 38.6 -> 32.9 us (155 MB, 4.7 TB/s), 2 x 4096 67.1 -> 57.5,
+// 2 x 1777 33.0 -> 29.2 (graph time over rotating buffers; separate q / k / v
+// buffers 37.0 -> 33.1 at 4096).
 #include "common.h"
 
 namespace dc {
@@ -40,7 +45,7 @@ struct QKArgs {
   int64_t fb, fl;      // frequency-table strides (floats) per batch, per position
   int L, H;
   int rows;            // B * L * H
-  int blocks_per_side;
+  int nsides;          // 1 (q), 2 (and k or v) or 3
   int flags;           // DC_QK_* bits
   int w_f32;           // weights are float32 (else the activation dtype)
   float eps, inv_d;
@@ -115,11 +120,16 @@ __device__ __forceinline__ float partner(float v) {
 template <int DT, int LPR, int NH>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(QKArgs a) {
   constexpr int RPW = 256 / LPR;   // lane groups per workgroup
-  const int side = blockIdx.x / a.blocks_per_side;
-  const int blk = blockIdx.x - side * a.blocks_per_side;
-  const int grp = blk * RPW + (int)threadIdx.x / LPR;   // rows NH * grp .. NH * grp + NH - 1
+  // q, k and v take turns 8 workgroups at a time (launch_qk pads each to a
+  // multiple of 8): workgroups go round-robin over 8 XCDs, so a token's q, k
+  // and v run close together in time and on one XCD
+  const int turn = blockIdx.x >> 3;
+  const int side = turn % a.nsides;
+  const unsigned blk = (unsigned)(turn / a.nsides) * 8u + (blockIdx.x & 7u);
+  const unsigned ugrp = blk * RPW + threadIdx.x / LPR;   // rows NH * grp .. NH * grp + NH - 1
   const int j = (int)threadIdx.x % LPR;
-  if (grp * NH >= a.rows) return;  // whole groups leave together: the lane exchanges stay inside live rows
+  if (ugrp >= (unsigned)a.rows / NH) return;  // whole groups leave together: the lane exchanges stay inside live rows
+  const int grp = (int)ugrp;
   const QKSide s = side == 0 ? a.s0 : (side == 1 ? a.s1 : a.s2);
   const int row0 = grp * NH;
   const int h0 = row0 % a.H;
@@ -219,14 +229,21 @@ template <int DT, int LPR, int NH>
 static int launch_qk(QKArgs& a, int nsides, hipStream_t st) {
   constexpr int RPW = 256 / LPR;
   const int groups = a.rows / NH;   // H % NH == 0, so rows % NH == 0
-  a.blocks_per_side = (groups + RPW - 1) / RPW;
-  hipLaunchKernelGGL((qk_norm_rope_kernel<DT, LPR, NH>), dim3(a.blocks_per_side * nsides), dim3(256), 0, st, a);
+  const unsigned blocks = (unsigned)((groups + RPW - 1) / RPW + 7) / 8 * 8;   // of one side
+  a.nsides = nsides;
+  hipLaunchKernelGGL((qk_norm_rope_kernel<DT, LPR, NH>), dim3(blocks * nsides), dim3(256), 0, st, a);
   return launch_status("dc_qk_norm_rope");
 }
 
+// Heads per lane group: 4 (fewer reads of the rotary matrices) while those
+// workgroups fill the chip's slots, 8 of 4 waves on each of 256 CUs; below
+// that 2, for twice the waves in flight. 24 heads of 128, q + k + v, graph
+// time over rotating buffers, 2 against 4: 512 tokens 7.8 / 8.4 us, 1024
+// 10.9 / 11.6; 3554 tokens 30.9 / 30.0, 4096 34.4 / 33.8, 8192 60.9 / 58.8.
 template <int DT, int LPR>
 static int launch_qk_heads(QKArgs& a, int nsides, hipStream_t st) {
-  if (a.H % 4 == 0) return launch_qk<DT, LPR, 4>(a, nsides, st);
+  constexpr int64_t SLOT_ROWS = 8 * 256 * (int64_t)(256 / LPR) * 4;   // rows those slots hold, 4 per lane group
+  if (a.H % 4 == 0 && (int64_t)a.rows * nsides >= SLOT_ROWS) return launch_qk<DT, LPR, 4>(a, nsides, st);
   if (a.H % 2 == 0) return launch_qk<DT, LPR, 2>(a, nsides, st);
   return launch_qk<DT, LPR, 1>(a, nsides, st);
 }
