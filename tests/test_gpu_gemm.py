@@ -572,3 +572,23 @@ def test_linear_one_call_refusals(gpu):
     m.bias = nn.Parameter(torch.zeros(64, device=gpu, dtype=torch.float64), requires_grad=False)
     with pytest.raises(TypeError):
         m(x)
+
+
+@pytest.mark.parametrize("k,group", [(256, 256), (512, 0), (48, 0)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_one_row_of_any_row_stride(gpu, k, group, dtype):
+    """A [1, K] input is taken whatever its row stride (a transposed column's
+    is 1, an expanded vector's may be anything below K, an odd-width buffer's
+    is misaligned), by the layer and by the two calls alike."""
+    m = _int8.Int8Linear(k, 64, group=group, device=gpu)
+    m.weight.copy_(torch.randint(-127, 128, (64, k), device=gpu))
+    m.scale_bits.copy_((torch.rand(64, device=gpu) * 1e-3).view(torch.int32))
+    x = torch.randn(1, k, device=gpu).to(dtype)
+    wide = torch.zeros(3, k + 1, device=gpu, dtype=dtype)
+    wide[0, :k] = x[0]
+    want = m(x)
+    for xi in (x.t().contiguous().t(), wide[:1, :k], torch.as_strided(x.clone(), (1, k), (0, 1)), x[0],
+               wide[None, :1, :k]):
+        assert torch.equal(m(xi).reshape(1, -1), want)
+        q, s = _int8.quantize_activation(xi.reshape(-1, k) if xi.dim() != 2 else xi, group)
+        assert torch.equal(m.matmul_quantized(q, s, dtype), want)

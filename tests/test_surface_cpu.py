@@ -237,6 +237,15 @@ def test_entry_points_refuse_host_tensors_before_any_launch():
 
 
 
+def test_one_row_keeps_its_own_length_as_the_row_stride():
+    """torch calls a one-row tensor contiguous whatever its row stride; the
+    kernels are told the row's length, so no such row is refused."""
+    x = torch.randn(256)
+    for row in (x.unsqueeze(1).t(), x.expand(1, 256), torch.cat((x, x[:1])).unsqueeze(0)[:, :256]):
+        got = _int8._rows(row)
+        assert got.stride() == (256, 1) and got.data_ptr() == row.data_ptr() and torch.equal(got[0], x)
+
+
 def test_quantize_and_dequantize_linears():
     model = nn.Sequential(nn.Linear(512, 256), nn.GELU(), nn.Linear(256, 64))
     assert D.quantize_linears(model, ["0", "2"], "cpu", group=0) == 2
