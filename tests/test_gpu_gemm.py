@@ -592,3 +592,23 @@ def test_one_row_of_any_row_stride(gpu, k, group, dtype):
         assert torch.equal(m(xi).reshape(1, -1), want)
         q, s = _int8.quantize_activation(xi.reshape(-1, k) if xi.dim() != 2 else xi, group)
         assert torch.equal(m.matmul_quantized(q, s, dtype), want)
+
+
+def test_forward_runs_an_overridden_matmul(gpu, monkeypatch):
+    """A forward goes through a subclass's or a patched matmul_quantized, and
+    through a patched quantize_activation."""
+    class Doubled(_int8.Int8Linear):
+        def matmul_quantized(self, q, s, dtype):
+            return super().matmul_quantized(q, s, dtype) * 2
+
+    m, sub = _int8.Int8Linear(256, 64, device=gpu), Doubled(256, 64, device=gpu)
+    for layer in (m, sub):
+        layer.weight.copy_(torch.arange(64 * 256, device=gpu).view(64, 256) % 255 - 127)
+        layer.scale_bits.copy_(torch.full((64,), 1e-3, device=gpu).view(torch.int32))
+    x = torch.randn(5, 256, device=gpu).half()
+    assert torch.equal(sub(x), m(x) * 2)
+    seen = []
+    real = _int8.quantize_activation
+    monkeypatch.setattr(_int8, "quantize_activation", lambda t, g: (seen.append(t.shape), real(t, g))[1])
+    want = sub(x)
+    assert torch.equal(m(x) * 2, want) and seen == [(5, 256)] * 2

@@ -246,6 +246,37 @@ def test_one_row_keeps_its_own_length_as_the_row_stride():
         assert got.stride() == (256, 1) and got.data_ptr() == row.data_ptr() and torch.equal(got[0], x)
 
 
+def test_forward_is_one_call_only_for_its_own_parts(monkeypatch):
+    """A subclass or a patch of what a forward is made of turns the one library
+    call off, for that layer only."""
+    layer = _int8.Int8Linear(256, 8)
+
+    class Sub(_int8.Int8Linear):
+        def matmul_quantized(self, q, s, dtype):
+            return super().matmul_quantized(q, s, dtype) * 2
+
+    class Scaled(_int8.Int8Linear):
+        @property
+        def scale(self):
+            return super().scale * 2
+
+    class Plain(_int8.Int8Linear):
+        pass
+
+    assert layer._one_call() and Plain(256, 8)._one_call()
+    assert not Sub(256, 8)._one_call() and not Scaled(256, 8)._one_call()
+    other = _int8.Int8Linear(256, 8)
+    other.matmul_quantized = lambda q, s, dtype: None
+    assert not other._one_call() and layer._one_call()
+    with monkeypatch.context() as mp:
+        mp.setattr(_int8.Int8Linear, "matmul_quantized", lambda self, q, s, dtype: None)
+        assert not layer._one_call()
+    with monkeypatch.context() as mp:
+        mp.setattr(_int8, "quantize_activation", lambda x, g: None)
+        assert not layer._one_call()
+    assert layer._one_call()
+
+
 def test_quantize_and_dequantize_linears():
     model = nn.Sequential(nn.Linear(512, 256), nn.GELU(), nn.Linear(256, 64))
     assert D.quantize_linears(model, ["0", "2"], "cpu", group=0) == 2
