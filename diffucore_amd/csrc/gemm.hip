@@ -1008,7 +1008,7 @@ static int device_cus() {
 // 8192 x 640 -> 640). Measured: FLUX's 512-row text MLP up 33.2 -> 30.5 us
 // and qkv 31.6 -> 27.8 us; the choice is unchanged on the other SD1.5 /
 // SDXL / FLUX shapes.
-// Tile class of a problem: DC_GEMM_PLAN_* (dc_w8a8_gemm_plan; pick_tile runs it on
+// Tile class of a problem: DC_GEMM_PLAN_* (dc_w8a8_gemm_plan; run_plan takes it for
 // the register-staged kernel where pick_dma has no tile).
 static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
   struct Cand { int bn, bm, per_cu; float eff; };
@@ -1083,10 +1083,68 @@ static DmaPick pick_dma(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
   return c192 < c256 ? DMA_192x256 : DMA_256x256;
 }
 
+// Split-K of the register-staged kernel, on 128 x 128 tiles, for problems
+// whose tiles fill at most a quarter of the device's workgroup slots (2 per
+// CU), with K >= 3072, or K >= 2048 for the tiniest (whatever tile plan_tile
+// would pick for the unsplit call: such problems leave most CUs idle either
+// way; measured, a fuller or shorter problem loses more to the
+// partials' round trip and the second launch than it gains): the largest
+// power of two S <= 8 with S * tiles <= slots and slices of at least 512
+// bytes of k, each slice a multiple of 128. Returns 1 for no split; *kslice
+// is the slice.
+static int splitk_plan(int64_t M, int64_t N, int64_t K, int* kslice) {
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t slots = 2 * (int64_t)device_cus();
+  // K >= 3072, or K >= 2048 when the tiles would fill at most 1/16 of the
+  // slots (SDXL's 154-row cross-attention K/V, 10-20 tiles: 14.5 -> 9.8-10.7
+  // us; at 80-96 tiles a 2048-deep split measured 30-50% slower)
+  if (K < 2048 || (K < 3072 && 16 * tiles > slots)) return 1;
+  if (4 * tiles > slots) return 1;
+  int s = 1;
+  while (s < 8 && 2 * s * tiles <= slots && K / (2 * s) >= 512) s *= 2;
+  if (s == 1) return 1;
+  const int64_t slice = ((K + s - 1) / s + 127) / 128 * 128;
+  *kslice = (int)slice;
+  return (int)((K + slice - 1) / slice);
+}
+
+// The same for a problem the DMA-fed kernel takes: its small tiles leave split-K
+// only the deepest products on the fewest rows (the partials and the second
+// launch cost about 4 us): 4 slices of 64 x 64 tiles from K = 8192 when those
+// tiles cover at most 3/4 of the CUs. 64 x 12288 -> 3072 23.8 -> 13.2 us,
+// 256 x 12288 -> 3072 25.2 -> 22.7; at 512 rows (64 x 128 tiles) 31.6 -> 35.5,
+// 154 x 2048 -> 1280 6.6 -> 8.5. K % 512 == 0 keeps the slices whole stages.
+static int dma_splits(int64_t M, int64_t N, int64_t K, int* kslice) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (K < 8192 || K % 512 || 4 * tiles > 3 * (int64_t)device_cus()) return 1;
+  *kslice = (int)(K / 4);
+  return 4;
+}
+
+// How a dc_w8a8_gemm call runs: the one answer that the call itself and the
+// workspace query share. dma: the DMA-fed kernel's tile, or DMA_NONE for the
+// register-staged kernel at `tile` (DC_GEMM_PLAN_*). splits > 1: k slices of
+// `kslice` bytes on that tile, their int32 partial sums in the workspace.
+struct RunPlan {
+  DmaPick dma;
+  int tile, splits, kslice;
+  size_t workspace(int64_t M, int64_t N) const { return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * 4 : 0; }
+};
+static RunPlan run_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, bool may_split) {
+  RunPlan r{pick_dma(M, N, K, lda, ldw), 0, 1, (int)K};
+  if (r.dma != DMA_NONE) {
+    if (may_split && (r.splits = dma_splits(M, N, K, &r.kslice)) > 1) r.dma = DMA_64x64;
+    return r;
+  }
+  r.tile = plan_tile(M, N, K, lda, ldw);
+  if (may_split && (r.splits = splitk_plan(M, N, K, &r.kslice)) > 1) r.tile = DC_GEMM_PLAN_128x128;
+  return r;
+}
+
 template <int OUT_DT, int BIAS_DT>
-static int pick_tile(GemmArgs p, hipStream_t st) {
+static int run_tile(const GemmArgs& p, const RunPlan& r, hipStream_t st) {
   const GroupArgs one{};
-  switch (pick_dma(p.M, p.N, p.K, p.lda, p.ldw)) {
+  switch (r.dma) {
     case DMA_256x256: return launch_gemm_dma<Dma256x256, OUT_DT, BIAS_DT>(p, one, st);
     case DMA_192x256: return launch_gemm_dma<Dma192x256, OUT_DT, BIAS_DT>(p, one, st);
     case DMA_128x128: return launch_gemm_dma<Dma128x128, OUT_DT, BIAS_DT>(p, one, st);
@@ -1096,7 +1154,7 @@ static int pick_tile(GemmArgs p, hipStream_t st) {
     case DMA_128x128K: return launch_gemm_dma<Dma128x128k, OUT_DT, BIAS_DT>(p, one, st);
     case DMA_NONE: break;
   }
-  switch (plan_tile(p.M, p.N, p.K, p.lda, p.ldw)) {
+  switch (r.tile) {
     case DC_GEMM_PLAN_192x256: return launch_gemm<Tile<2, 4, 3, 2, 1>, OUT_DT, BIAS_DT>(p, st);
     case DC_GEMM_PLAN_192x128: return launch_gemm<Tile<2, 2, 3, 2, 1>, OUT_DT, BIAS_DT>(p, st);
     case DC_GEMM_PLAN_128x128: return launch_gemm<Tile<2, 2, 2, 2, 1>, OUT_DT, BIAS_DT>(p, st);
@@ -1105,12 +1163,12 @@ static int pick_tile(GemmArgs p, hipStream_t st) {
 }
 
 template <int OUT_DT>
-static int dispatch_bias(GemmArgs p, int bias_dtype, hipStream_t st) {
+static int dispatch_bias(const GemmArgs& p, const RunPlan& r, int bias_dtype, hipStream_t st) {
   switch (bias_dtype) {
-    case DC_NONE: return pick_tile<OUT_DT, DC_NONE>(p, st);
-    case DC_F16: return pick_tile<OUT_DT, DC_F16>(p, st);
-    case DC_BF16: return pick_tile<OUT_DT, DC_BF16>(p, st);
-    case DC_F32: return pick_tile<OUT_DT, DC_F32>(p, st);
+    case DC_NONE: return run_tile<OUT_DT, DC_NONE>(p, r, st);
+    case DC_F16: return run_tile<OUT_DT, DC_F16>(p, r, st);
+    case DC_BF16: return run_tile<OUT_DT, DC_BF16>(p, r, st);
+    case DC_F32: return run_tile<OUT_DT, DC_F32>(p, r, st);
     default: return fail(DC_EINVAL, "dc_w8a8_gemm: bad bias_dtype");
   }
 }
@@ -1146,46 +1204,6 @@ static int rescale_bias(const int32_t* acc, int64_t lda, const float* sx, const 
   }
 }
 
-// Split-K plan for problems whose 128 x 128 tiles fill at most a quarter of
-// the device's workgroup slots (2 per CU), with K >= 3072, or K >= 2048 for
-// the tiniest (whatever tile
-// plan_tile would pick for the unsplit call: such problems leave most CUs
-// idle either way; measured, a fuller or shorter problem loses more to the
-// partials' round trip and the second launch than it gains): the largest
-// power of two S <= 8 with S * tiles <= slots and slices of at least 512
-// bytes of k, each slice a multiple of 128. Returns 1 for no split; *kslice
-// is the slice.
-static int splitk_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int* kslice) {
-  *kslice = (int)K;
-  (void)lda; (void)ldw;
-  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  const int64_t slots = 2 * (int64_t)device_cus();
-  // K >= 3072, or K >= 2048 when the tiles would fill at most 1/16 of the
-  // slots (SDXL's 154-row cross-attention K/V, 10-20 tiles: 14.5 -> 9.8-10.7
-  // us; at 80-96 tiles a 2048-deep split measured 30-50% slower)
-  if (K < 2048 || (K < 3072 && 16 * tiles > slots)) return 1;
-  if (4 * tiles > slots) return 1;
-  int s = 1;
-  while (s < 8 && 2 * s * tiles <= slots && K / (2 * s) >= 512) s *= 2;
-  if (s == 1) return 1;
-  const int64_t slice = ((K + s - 1) / s + 127) / 128 * 128;
-  *kslice = (int)slice;
-  return (int)((K + slice - 1) / slice);
-}
-
-// The same for a problem the DMA-fed kernel takes: its small tiles leave split-K
-// only the deepest products on the fewest rows (the partials and the second
-// launch cost about 4 us): 4 slices of 64 x 64 tiles from K = 8192 when those
-// tiles cover at most 3/4 of the CUs. 64 x 12288 -> 3072 23.8 -> 13.2 us,
-// 256 x 12288 -> 3072 25.2 -> 22.7; at 512 rows (64 x 128 tiles) 31.6 -> 35.5,
-// 154 x 2048 -> 1280 6.6 -> 8.5. K % 512 == 0 keeps the slices whole stages.
-static int dma_splits(int64_t M, int64_t N, int64_t K, int* kslice) {
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (K < 8192 || K % 512 || 4 * tiles > 3 * (int64_t)device_cus()) return 1;
-  *kslice = (int)(K / 4);
-  return 4;
-}
-
 }  // namespace dc
 
 using namespace dc;
@@ -1202,9 +1220,7 @@ extern "C" int dc_w8a8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t lda, i
 extern "C" size_t dc_w8a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 16 || lda < K || ldw < K || lda % 16 || ldw % 16) return 0;
   if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-  int kslice = 0;
-  const int s = splitk_plan(M, N, K, lda, ldw, &kslice);
-  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * 4 : 0;
+  return run_plan(M, N, K, lda, ldw, true).workspace(M, N);
 }
 
 extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64_t ldw, const float* sx,
@@ -1234,39 +1250,32 @@ extern "C" int dc_w8a8_gemm(const int8_t* a, int64_t lda, const int8_t* w, int64
     return fail(DC_EINVAL, "dc_w8a8_gemm: bad out_dtype");
   if (bias_dtype != DC_NONE && bias_dtype != DC_F16 && bias_dtype != DC_BF16 && bias_dtype != DC_F32)
     return fail(DC_EINVAL, "dc_w8a8_gemm: bad bias_dtype");
+  RunPlan r = run_plan(M, N, K, lda, ldw, out_dtype != DC_I32 && workspace && aligned16(workspace));
+  if (ws_bytes < r.workspace(M, N)) r = run_plan(M, N, K, lda, ldw, false);
   // split-K into the workspace (int32 partials), then the epilogue over their sum
-  int kslice = 0;
-  int ks = (out_dtype != DC_I32 && workspace) ? splitk_plan(M, N, K, lda, ldw, &kslice) : 1;
-  const bool dma = ks > 1 && pick_dma(M, N, K, lda, ldw) != DMA_NONE;
-  if (dma) {   // the caller's workspace holds splitk_plan's slices
-    const int n = dma_splits(M, N, K, &kslice);
-    ks = ks >= n ? n : 1;
-  }
-  if (ks > 1 && ws_bytes >= (size_t)ks * (size_t)M * (size_t)N * 4 && aligned16(workspace)) {
+  if (r.splits > 1) {
     GemmArgs q = p;
     q.sx = nullptr; q.sw = nullptr; q.bias = nullptr;
     q.out = workspace;
     q.ldo = N;
     q.vec_out = N % 4 == 0;
     q.vec16 = N % 4 == 0;
-    q.ksplit = ks;
-    q.kslice = kslice;
+    q.ksplit = r.splits;
+    q.kslice = r.kslice;
     q.split_stride = M * N;
-    if (int e = dma ? launch_gemm_dma<Dma64x64, DC_I32, DC_NONE>(q, GroupArgs{}, st)
-                    : launch_gemm<Tile<2, 2, 2, 2, 1>, DC_I32, DC_NONE>(q, st))
-      return e;
+    if (int e = run_tile<DC_I32, DC_NONE>(q, r, st)) return e;
     const int32_t* acc = static_cast<const int32_t*>(workspace);
     switch (out_dtype) {
-      case DC_F16: return rescale_bias<DC_F16>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, ks, M * N);
-      case DC_BF16: return rescale_bias<DC_BF16>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, ks, M * N);
-      default: return rescale_bias<DC_F32>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, ks, M * N);
+      case DC_F16: return rescale_bias<DC_F16>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, r.splits, M * N);
+      case DC_BF16: return rescale_bias<DC_BF16>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, r.splits, M * N);
+      default: return rescale_bias<DC_F32>(acc, N, sx, sw, bias, bias_dtype, out, ldo, M, N, st, r.splits, M * N);
     }
   }
   switch (out_dtype) {
-    case DC_I32: return pick_tile<DC_I32, DC_NONE>(p, st);
-    case DC_F16: return dispatch_bias<DC_F16>(p, bias_dtype, st);
-    case DC_BF16: return dispatch_bias<DC_BF16>(p, bias_dtype, st);
-    case DC_F32: return dispatch_bias<DC_F32>(p, bias_dtype, st);
+    case DC_I32: return run_tile<DC_I32, DC_NONE>(p, r, st);
+    case DC_F16: return dispatch_bias<DC_F16>(p, r, bias_dtype, st);
+    case DC_BF16: return dispatch_bias<DC_BF16>(p, r, bias_dtype, st);
+    case DC_F32: return dispatch_bias<DC_F32>(p, r, bias_dtype, st);
     default: return fail(DC_EINVAL, "dc_w8a8_gemm: bad out_dtype");
   }
 }

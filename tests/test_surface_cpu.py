@@ -320,10 +320,15 @@ def test_argument_checks_fail_before_any_launch():
     assert b"K" in so.dc_last_error()
     assert so.dc_w8a8_gemm(16, 32, 16, 32, 16, 16, None, 7, 16, _lib.BF16, 8, 4, 8, 32, None, 0, None) == 1
     # split-K workspace: small M with long K splits (FLUX text MLP down: 4 slices of int32 partials), big M does not
-    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 12288, 12288, 12288) == 4 * 512 * 3072 * 4
+    # what the call splits into, and nothing where it runs unsplit (256 CUs)
+    assert so.dc_w8a8_gemm_workspace_bytes(64, 3072, 12288, 12288, 12288) == 4 * 64 * 3072 * 4
+    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 12288, 12288, 12288) == 0
     assert so.dc_w8a8_gemm_workspace_bytes(4096, 3072, 12288, 12288, 12288) == 0
-    assert so.dc_w8a8_gemm_workspace_bytes(154, 1280, 2048, 2048, 2048) == 4 * 154 * 1280 * 4   # 20 tiles
-    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 2048, 2048, 2048) == 0   # 96 tiles: no 2048-deep split
+    assert so.dc_w8a8_gemm_workspace_bytes(154, 1280, 2048, 2048, 2048) == 0
+    assert so.dc_w8a8_gemm_workspace_bytes(154, 1280, 2064, 2064, 2064) == 4 * 154 * 1280 * 4   # 20 register-staged
+    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 2064, 2064, 2064) == 0   # 96 tiles: no 2048-deep split
+    codes, scales = 512 * 3072, 512 * 4                                         # of a layer: no unused partials
+    assert so.dc_w8a8_linear_scratch_bytes(512, 3072, 3072, 3072) == codes + scales
     assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 100, 112, 112) == 0
     assert so.dc_int8_attn_workspace_bytes(1, 24, 4608, 4608, 128) > 24 * 4608 * 128
     assert so.dc_int8_attn_workspace_bytes(1, 1, 1, 1, 200) == 0
