@@ -126,9 +126,9 @@ class HotPath:
         assert all(isinstance(op[1], _int8.Int8Linear) for op in self.ops if op[0] == "gemm")
         assert all(isinstance(la, _int8.Int8Linear) for op in self.ops if op[0] == "group" for la in op[1])
         self.total_ops = sum(op[3] for op in self.ops)
-        # which GEMM kernel each launch runs (dc_w8a8_gemm_plan; grouped
+        # which GEMM kernel each launch runs (dc_w8a8_gemm_kernel; grouped
         # launches always run the DMA-fed 256 x 256 kernel)
-        self.plans = [_int8.gemm_plan(op[2].shape[0], op[1].out_features, op[1].in_features) if op[0] == "gemm"
+        self.plans = [_int8.gemm_kernel(op[2].shape[0], op[1].out_features, op[1].in_features)[0] if op[0] == "gemm"
                       else "dma_256x256" if op[0] == "group" else None for op in self.ops]
         self.ws = None
 
@@ -136,7 +136,7 @@ class HotPath:
         """One step. With ``recs`` (a list), HIP events on torch's current
         stream (where every kernel of this package is launched) bracket each
         quantize, GEMM and attention call and are appended as
-        ``(kind, start, end, ops, bytes, gemm plan or None)``."""
+        ``(kind, start, end, ops, bytes, gemm kernel or None)``."""
         from diffucore_amd import _int8, attention_bhld
         q, k, v = self.qkv
         if recs is None:
@@ -186,7 +186,7 @@ class HotPath:
 
 def summarize(recs):
     """Per-kernel totals over recorded events; GEMM launches are also totalled
-    per kernel plan (``gemm_<plan>``, from dc_w8a8_gemm_plan)."""
+    per kernel (``gemm_<kernel>``, from dc_w8a8_gemm_kernel)."""
     out = {}
     for kind, a, b, ops, nbytes, plan in recs:
         for key in (kind, f"gemm_{plan}") if plan else (kind,):
@@ -575,7 +575,7 @@ def gemm_vendor_ab(dev):
             return round(ops / (ms * 1e-3) / 1e12, 1)
 
         print(json.dumps({"kind": "gemm_vs_vendor", "shape": name, "M": M, "K": K, "N": N,
-                          "plan": __import__("diffucore_amd")._int8.gemm_plan(M, N, K),
+                          "plan": __import__("diffucore_amd")._int8.gemm_kernel(M, N, K)[0],
                           "torch_int_mm_ms": round(ms_v, 4), "torch_int_mm_TOPS": tops(ms_v),
                           "torch_int_mm_rescale_ms": round(ms_vr, 4),
                           "dc_int32_ms": round(ms_i, 4), "dc_int32_TOPS": tops(ms_i),
@@ -710,7 +710,7 @@ def shapes_report(dev):
         gbytes = M * K + N * K + 4 * (M + N) + N * m.bias.element_size() + M * N * x.element_size()
         tops = ops / (ms_gg * 1e-3) / 1e12
         print(json.dumps({"kind": "w8a8_linear", "shape": name, "M": M, "K": K, "N": N, "group": group,
-                          "dtype": str(dt)[6:], "plan": __import__("diffucore_amd")._int8.gemm_plan(M, N, K),
+                          "dtype": str(dt)[6:], "plan": __import__("diffucore_amd")._int8.gemm_kernel(M, N, K)[0],
                           "gemm_ms": round(ms_g, 4), "gemm_gpu_ms": round(ms_gg, 4), "TOPS": round(tops, 1),
                           "pct_int8_peak": round(100 * tops / INT8_PEAK_TOPS, 2),
                           "gemm_bytes": gbytes, "gemm_GBps": round(gbytes / (ms_gg * 1e-3) / 1e9, 1),
@@ -1027,10 +1027,9 @@ def main():
         traffic_src["matches_current_source"] = tj.get("kernel_source_sha256") == gemm_source_sha256()
         if traffic_src["matches_current_source"]:
             traffic = tj.get("hbm_bytes_per_launch")
-    roofline = {"kernel": "w8a8_gemm_dma_kernel (256x256 tiles, 4 waves, operands loaded straight into LDS): the "
-                          f"{g['launches'] // args.steps} FLUX-step launches it runs (img MLP up; the double blocks' "
-                          "img + txt qkv, proj and MLP down, each pair as one grouped launch; single linear1 and "
-                          "linear2)",
+    roofline = {"kernel": "w8a8_gemm_dma_kernel (256x256 tiles, 8 waves, operands loaded straight into LDS): the "
+                          f"{g['launches'] // args.steps} FLUX-step launches it runs (the double blocks' img + txt "
+                          "pairs that share a grouped launch, and the layers whose own tile it is)",
                 "bound": "mfma", "achieved": round(achieved, 1), "peak": INT8_PEAK_TOPS, "unit": "TOP/s",
                 "frac": round(achieved / INT8_PEAK_TOPS, 4), "traffic": traffic, "traffic_source": traffic_src,
                 "algorithmic_ops_per_launch": int(ops_per_launch),

@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime first)
 LIB_PATH = Path(__file__).resolve().parent / "libdiffucore_amd.so"
 
 F16, BF16, F32, I32, NONE = 0, 1, 2, 3, -1
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _DTYPE = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32, torch.int32: I32}
 
@@ -34,6 +34,7 @@ _SIGS = {
     "dc_w8a8_linear_scratch_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _I64]),
     "dc_w8a8_gemm_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64]),
     "dc_w8a8_gemm_plan": (_I, [_I64, _I64, _I64, _I64, _I64]),
+    "dc_w8a8_gemm_kernel": (_I, [_I64, _I64, _I64, _I64, _I64, ctypes.POINTER(_I)]),
     "dc_w8a8_gemm_grouped": (_I, [_P, _I, _I64, _I64, _I, _I, _P]),
     "dc_w8a8_gemm_grouped_gated": (_I, [_P, _P, _I, _I64, _I64, _I, _I, _P]),
     "dc_w8a8_gemm_group_plan": (_I, [ctypes.POINTER(_I64), _I, _I64, _I64]),
@@ -87,12 +88,12 @@ def lib():
     except OSError as e:
         _load_error = f"cannot load {LIB_PATH.name}: {e}"
         return None
+    if so.dc_abi_version() != ABI_VERSION:   # before the symbols: an older library lacks some
+        _load_error = f"{LIB_PATH.name} ABI {so.dc_abi_version()} != {ABI_VERSION}: rebuild it"
+        return None
     for name, (res, args) in _SIGS.items():
         fn = getattr(so, name)
         fn.restype, fn.argtypes = res, args
-    if so.dc_abi_version() != ABI_VERSION:
-        _load_error = f"{LIB_PATH.name} ABI {so.dc_abi_version()} != {ABI_VERSION}: rebuild it"
-        return None
     return so
 
 

@@ -11,9 +11,10 @@
 //   workgroup tile  BN x BM = (32*WN*FN) x (32*WM*FM), WN x WM waves
 //   wave tile       (32*FN) x (32*FM) = FN x FM MFMA blocks of 32 x 32
 // Two kernels:
-//   w8a8_gemm_dma_kernel  K % 64 == 0 (every layer width of the SD1.5, SDXL
-//     and FLUX models): operands loaded straight into an LDS ring; seven tiles
-//     from 64 x 64 to 256 x 256, chosen by pick_dma.
+//   w8a8_gemm_dma_kernel  K % 128 == 0, and K = 64 (mod 128) below 1024 (every
+//     layer width of the SD1.5, SDXL and FLUX models): operands loaded
+//     straight into an LDS ring; seven tiles from 64 x 64 to 256 x 256, chosen
+//     by pick_dma.
 //   w8a8_gemm_kernel      the other K (multiples of 16) and row strides past
 //     the DMA's 32-bit offsets: 128 k-bytes per LDS stage, two stages; 256 x
 //     256 tiles on 8 waves (2 along n x 4 along m, each 128 x 64), 192 x 256
@@ -1063,7 +1064,16 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
 // K = 64 (mod 128): 64-byte stages at 128 x 128, 3 workgroups per CU; 8192 x
 // 320 -> 1280 with float32 out 18.4 -> 12.7 us. Only below K = 1024: deeper
 // ones would want the larger tiles of the register-staged kernel.
-enum DmaPick { DMA_NONE, DMA_256x256, DMA_192x256, DMA_128x128, DMA_128x128D, DMA_64x128, DMA_64x64, DMA_128x128K };
+enum DmaPick {
+  DMA_NONE = 0,
+  DMA_256x256 = DC_GEMM_DMA_256x256,
+  DMA_192x256 = DC_GEMM_DMA_192x256,
+  DMA_128x128 = DC_GEMM_DMA_128x128,
+  DMA_128x128D = DC_GEMM_DMA_128x128_8W,
+  DMA_64x128 = DC_GEMM_DMA_64x128,
+  DMA_64x64 = DC_GEMM_DMA_64x64,
+  DMA_128x128K = DC_GEMM_DMA_128x128_K64
+};
 static DmaPick pick_dma(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
   if (K % 64 || 256 * lda >= (int64_t(1) << 31) || 256 * ldw >= (int64_t(1) << 31)) return DMA_NONE;
   if (K % 128) return K < 1024 ? DMA_128x128K : DMA_NONE;
@@ -1122,7 +1132,7 @@ static int dma_splits(int64_t M, int64_t N, int64_t K, int* kslice) {
 }
 
 // How a dc_w8a8_gemm call runs: the one answer that the call itself and the
-// workspace query share. dma: the DMA-fed kernel's tile, or DMA_NONE for the
+// workspace and kernel queries share. dma: the DMA-fed kernel's tile, or DMA_NONE for the
 // register-staged kernel at `tile` (DC_GEMM_PLAN_*). splits > 1: k slices of
 // `kslice` bytes on that tile, their int32 partial sums in the workspace.
 struct RunPlan {
@@ -1215,6 +1225,18 @@ extern "C" int dc_w8a8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t lda, i
     return -1;
   }
   return plan_tile(M, N, K, lda, ldw);
+}
+
+extern "C" int dc_w8a8_gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int* slices) {
+  clear_error();
+  if (M <= 0 || N <= 0 || K <= 0 || K % 16 || lda < K || ldw < K || lda % 16 || ldw % 16 || M > 0x7fffffff ||
+      N > 0x7fffffff || K > 0x7fffffff) {
+    set_error("dc_w8a8_gemm_kernel: no kernel takes this shape");
+    return -1;
+  }
+  const RunPlan r = run_plan(M, N, K, lda, ldw, true);
+  if (slices) *slices = r.splits;
+  return r.dma != DMA_NONE ? (int)r.dma : r.tile;
 }
 
 extern "C" size_t dc_w8a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {

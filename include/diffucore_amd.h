@@ -179,13 +179,13 @@ size_t dc_w8a8_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t ldw
 
 /*
  * Tile class of a dc_w8a8_gemm problem on the current device: one of the
- * DC_GEMM_PLAN_* codes, or -1 for a shape it rejects. Classes are chosen by how
- * full the last round of workgroups keeps the device. K that is not a multiple
- * of 64 runs exactly that tile; other K run on the DMA-fed kernel, whose own
- * rule may take another tile of it. A problem of class DMA_256x256 is one that
- * dc_w8a8_gemm_grouped(_gated) takes without losing to dc_w8a8_gemm. No
+ * DC_GEMM_PLAN_* codes, or -1 for a shape it rejects, chosen by how full the
+ * last round of workgroups keeps the device. It is the register-staged
+ * kernel's tile where that kernel runs the problem; what runs is
+ * dc_w8a8_gemm_kernel's answer. A single gated problem (K % 256 == 0) goes to
+ * dc_w8a8_gemm_grouped_gated where its class is DMA_256x256. No
  * counterpart in the reference (its GEMMs come from torch._int_mm and one
- * CUTLASS configuration, _int8.py:200-276); for profiling, dispatch and tests.
+ * CUTLASS configuration, _int8.py:200-276); for dispatch and tests.
  */
 enum {
   DC_GEMM_PLAN_256x256 = 0,      /* 8 waves, 128 x 64 wave tiles, register-staged loads */
@@ -195,6 +195,26 @@ enum {
   DC_GEMM_PLAN_192x128 = 4       /* 192 (n) x 128 (m) on 4 waves, 96 x 64 wave tiles, 1 workgroup per CU */
 };
 int dc_w8a8_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw);
+
+/*
+ * The kernel dc_w8a8_gemm runs a problem on, given the workspace it asks for
+ * (dc_w8a8_gemm_workspace_bytes), on the current device: a DC_GEMM_DMA_* code
+ * for a tile (n x m) of the DMA-fed kernel, a DC_GEMM_PLAN_* code for one of
+ * the register-staged kernel, or -1 for a shape it rejects. *slices (may be
+ * NULL): the k slices it splits into, 1 for none (an int32 output never
+ * splits). No counterpart in the reference (_int8.py:200-276); for profiling
+ * and tests.
+ */
+enum {
+  DC_GEMM_DMA_256x256 = 16,    /* 8 waves of 64 x 128; also the grouped launches' */
+  DC_GEMM_DMA_192x256 = 17,    /* 8 waves of 96 x 64 */
+  DC_GEMM_DMA_128x128 = 18,    /* 4 waves of 64 x 64, 2 workgroups per CU */
+  DC_GEMM_DMA_128x128_8W = 19, /* 8 waves of 64 x 32, 1 per CU */
+  DC_GEMM_DMA_64x128 = 20,     /* 8 waves of 32 x 32, 2 per CU */
+  DC_GEMM_DMA_64x64 = 21,      /* 4 waves of 32 x 32, 3 per CU */
+  DC_GEMM_DMA_128x128_K64 = 22 /* 4 waves of 64 x 64, 64-byte stages, 3 per CU */
+};
+int dc_w8a8_gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int* slices);
 
 /*
  * Grouped W8A8 GEMM: up to DC_GEMM_MAX_GROUP problems that share N, K, the

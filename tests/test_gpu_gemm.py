@@ -107,7 +107,7 @@ def test_cfg1_sd15_linear_exact(gpu):
     scales (quantized on the CPU) equal the oracle's weight quantizer; the
     activation codes and scales and the fp32 output equal the oracle's
     quantize -> int_mm -> rescale bit for bit. K = 320 = 2 x 128 + 64 runs the
-    register-staged kernel's masked k tail."""
+    DMA-fed kernel's 64-byte stages."""
     g = torch.Generator().manual_seed(0)
     x = torch.randn(8192, 320, generator=g)
     idx = torch.randperm(320, generator=g)[:2]
@@ -121,6 +121,7 @@ def test_cfg1_sd15_linear_exact(gpu):
     assert np.array_equal(m.weight.cpu().numpy(), wq)
     assert np.array_equal(m.scale.cpu().numpy().view(np.uint32), np.asarray(ws, np.float32).view(np.uint32))
     assert _int8.gemm_plan(8192, 1280, 320) != "dma_256x256"
+    assert _int8.gemm_kernel(8192, 1280, 320) == ("dma_128x128_k64", 1)
     xg = x.to(gpu)
     qa, sa = _int8.quantize_activation(xg, 0)
     oq, osc = OQ.quantize_activation(x.numpy(), 0)
@@ -141,20 +142,23 @@ def test_short_input(gpu):
     assert rel_l2(np32(_int8.Int8Linear.from_linear(lin)(x)), np32(lin(x))) < 0.02
 
 
-# shapes that select each kernel (by how full the last round of tiles is on a
-# 256-CU device, and K % 256 for the DMA-fed 256 x 256 kernel), with M, N and
-# K tails among them
-TILE_SHAPES = [((4096, 12288, 512), "dma_256x256"), ((4608, 3072, 256), "dma_256x256"),
-               ((4096, 12288, 272), "256x256"), ((4096, 3072, 512), "192x256"),
-               ((4000, 3000, 272), "192x256"), ((512, 3072, 512), "128x128"), ((4001, 12200, 768), "dma_256x256"),
-               ((512, 12288, 3072), "192x128"), ((500, 12200, 336), "192x128")]
+# shapes of each tile class (by how full the last round of tiles is on a
+# 256-CU device, and K % 256 for DMA_256x256) and the kernel that runs them,
+# with M, N and K tails among them; the register-staged kernel at each of its
+# four tiles
+TILE_SHAPES = [((4096, 12288, 512), "dma_256x256", "dma_192x256"), ((4608, 3072, 256), "dma_256x256", "dma_128x128"),
+               ((4096, 12288, 272), "256x256", "256x256"), ((4096, 3072, 512), "192x256", "dma_192x256"),
+               ((4000, 3000, 272), "192x256", "192x256"), ((512, 3072, 512), "128x128", "dma_64x128"),
+               ((4001, 12200, 768), "dma_256x256", "dma_192x256"), ((512, 12288, 3072), "192x128", "dma_128x128"),
+               ((500, 12200, 336), "192x128", "192x128"), ((500, 3070, 528), "128x128", "128x128"),
+               ((2500, 6140, 1024), "dma_256x256", "dma_256x256")]
 
 
-@pytest.mark.parametrize("mnk,plan", TILE_SHAPES)
-def test_every_tile_configuration(gpu, mnk, plan):
+@pytest.mark.parametrize("mnk,plan,kernel", TILE_SHAPES)
+def test_every_tile_configuration(gpu, mnk, plan, kernel):
     m, n, k = mnk
     if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
-        assert _int8.gemm_plan(m, n, k) == plan
+        assert _int8.gemm_plan(m, n, k) == plan and _int8.gemm_kernel(m, n, k) == (kernel, 1)
     q, w, sx, sw = _qw(m, n, k, 9)
     bias = (torch.randn(n, generator=torch.Generator().manual_seed(9)) * 0.5).to(torch.bfloat16)
     lin = _int8.Int8Linear(k, n, bias=True, group=0, device=gpu)
@@ -478,24 +482,28 @@ def test_multi_round_grouped_gemm_bit_exact(gpu, ms, n, k, dtype, bias_dtype):
     assert all(torch.equal(a, c) for a, c in zip(_int8._gemm_grouped(items, dtype), outs))
 
 
-# The DMA-fed kernel's tiles (64 x 64, 64 x 128, 128 x 128 one and two per CU,
-# 192 x 256, 256 x 256; 128 x 128 with 64-byte stages for K = 64 mod 128) at
-# whole and ragged edges, with fewer k stages than the ring holds, as many, and
-# one or two more; the last ones leave K % 64 or its depth to the
-# register-staged kernel.
-DMA_EDGES = [(1, 8, 128), (64, 64, 256), (65, 130, 384), (154, 2560, 512), (129, 513, 128), (512, 3071, 640),
-             (500, 3072, 1280), (1000, 2048, 256), (1025, 2049, 384), (2048, 1281, 512), (2047, 3840, 128),
-             (2000, 3840, 640), (4096, 3072, 1024), (4095, 3001, 384), (2560, 16384, 256), (2500, 16380, 384),
-             (7904, 1920, 640), (1, 4, 64), (130, 260, 192), (8192, 1280, 320), (3000, 1284, 576), (100, 100, 960),
-             (257, 300, 1088), (300, 200, 48)]
+# The DMA-fed kernel's tiles at whole and ragged edges, with fewer k stages
+# than the ring holds, as many, and one or two more; the last ones leave K % 64
+# or its depth to the register-staged kernel. The tile each case runs on is the
+# one before it in the list (256 CUs).
+DMA_EDGES = [("dma_64x64", [(1, 8, 128), (64, 64, 256), (65, 130, 384), (154, 2560, 512), (129, 513, 128)]),
+             ("dma_64x128", [(512, 3071, 640), (500, 3072, 1280), (1000, 2048, 256)]),
+             ("dma_128x128_8w", [(1025, 2049, 384), (2048, 1281, 512)]),
+             ("dma_128x128", [(2047, 3840, 128), (2000, 3840, 384), (7904, 1920, 640)]),
+             ("dma_192x256", [(4096, 3072, 1024), (4095, 3001, 384), (2560, 16384, 256), (2500, 16380, 384)]),
+             ("dma_256x256", [(2304, 6144, 1024), (2500, 6140, 1536)]),
+             ("dma_128x128_k64", [(1, 4, 64), (130, 260, 192), (8192, 1280, 320), (3000, 1284, 576), (100, 100, 960)]),
+             ("128x128", [(257, 300, 1088), (300, 200, 48)])]
 
 
-@pytest.mark.parametrize("mnk", DMA_EDGES)
-def test_dma_tiles_bit_exact(gpu, mnk):
+@pytest.mark.parametrize("mnk,kernel", [(mnk, kernel) for kernel, shapes in DMA_EDGES for mnk in shapes])
+def test_dma_tiles_bit_exact(gpu, mnk, kernel):
     """Every tile and edge against the vendor's int32 product and the rescale
     expression in torch ops, from operands that are slices of wider rows
     (strides above K) into an output of every type."""
     m, n, k = mnk
+    if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
+        assert _int8.gemm_kernel(m, n, k, k + 32, k + 32) == (kernel, 1)
     g = torch.Generator(device=gpu).manual_seed(m * 7 + n + k)
     wide = k + 32
     q = torch.randint(-128, 128, (m, wide), generator=g, device=gpu, dtype=torch.int8)[:, 16:16 + k]

@@ -476,6 +476,42 @@ def test_gemm_plan_choice_without_a_gpu():
     assert [_int8.gemm_plan(4608, 21504, 3072), _int8.gemm_plan(512, 9216, 3072)] == ["dma_256x256", "192x128"]
 
 
+def test_gemm_kernel_names_what_runs():
+    """dc_w8a8_gemm_kernel: the DMA-fed kernel's own tile where it takes the
+    problem (K % 128 == 0, or K = 64 mod 128 below 1024, row strides below
+    2^23), else the class's register-staged tile, with the k slices (256 CUs)."""
+    kernel = _int8.gemm_kernel
+    assert kernel(4608, 21504, 3072) == ("dma_256x256", 1)      # linear1
+    assert kernel(4096, 9216, 3072) == ("dma_192x256", 1)       # image qkv
+    assert kernel(512, 12288, 3072) == ("dma_128x128", 1)       # text MLP up: class 192x128
+    assert kernel(2048, 1280, 1280) == ("dma_128x128_8w", 1)
+    assert kernel(512, 3072, 3072) == ("dma_64x128", 1)
+    assert kernel(154, 2560, 2048) == ("dma_64x64", 1)
+    assert kernel(8192, 1280, 320) == ("dma_128x128_k64", 1)
+    assert kernel(8192, 1280, 1088) == (_int8.gemm_plan(8192, 1280, 1088), 1)
+    assert kernel(154, 640, 4112) == ("128x128", 7)
+    assert kernel(4096, 9216, 3072, lda=1 << 23) == (_int8.gemm_plan(4096, 9216, 3072, lda=1 << 23), 1)
+    for m, n, k in ((64, 3072, 12288), (154, 640, 4112), (512, 3072, 3072)):
+        slices = kernel(m, n, k)[1]
+        want = slices * m * n * 4 if slices > 1 else 0
+        assert _lib.lib().dc_w8a8_gemm_workspace_bytes(m, n, k, k, k) == want
+    for bad in ((0, 1, 16), (1, 1, 20), (1 << 31, 16, 16)):
+        with pytest.raises(RuntimeError, match="no kernel takes"):
+            kernel(*bad)
+
+
+def test_an_older_library_is_refused_by_its_version(monkeypatch, tmp_path):
+    """A library of another ABI version is reported as one to rebuild, also
+    when it lacks symbols of this one."""
+    src = tmp_path / "old.c"
+    src.write_text("int dc_abi_version(void) { return 1; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "old.so"), str(src)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "old.so")
+    monkeypatch.setattr(_lib, "_load_error", "")
+    assert _lib.lib.__wrapped__() is None
+    assert "ABI 1 != " in _lib._load_error and "rebuild" in _lib._load_error
+
+
 @pytest.mark.skipif(not _lib.LIB_PATH.exists(), reason="library not built")
 def test_attention_work_split_without_a_gpu():
     """The attention work split runs on the host (512 resident workgroups, 2
