@@ -1118,17 +1118,57 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, int* kslice) {
   return (int)((K + slice - 1) / slice);
 }
 
-// The same for a problem the DMA-fed kernel takes: its small tiles leave split-K
-// only the deepest products on the fewest rows (the partials and the second
-// launch cost about 4 us): 4 slices of 64 x 64 tiles from K = 8192 when those
-// tiles cover at most 3/4 of the CUs. 64 x 12288 -> 3072 23.8 -> 13.2 us,
-// 256 x 12288 -> 3072 25.2 -> 22.7; at 512 rows (64 x 128 tiles) 31.6 -> 35.5,
-// 154 x 2048 -> 1280 6.6 -> 8.5. K % 512 == 0 keeps the slices whole stages.
-static int dma_splits(int64_t M, int64_t N, int64_t K, int* kslice) {
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (K < 8192 || K % 512 || 4 * tiles > 3 * (int64_t)device_cus()) return 1;
-  *kslice = (int)(K / 4);
-  return 4;
+// The same for a problem the DMA-fed kernel takes: slices of whole 128-byte
+// stages (the last may be shorter), and the tile they run on.
+// A split costs the partials' round trip and a second launch, about 4 us, so
+// nothing below K = 4096 splits. From there a product on few rows is a few
+// long chains of k stages on an idle chip.
+//   s64, s64x128, s128: the slices that give each CU one workgroup of that
+//     tile, of at least 1280 (1792) bytes of k, as a shorter chain no longer
+//     pays for its partials.
+//   M <= 64 (weights read once, little to add up): two 64 x 64 workgroups per
+//     CU where one each leaves the chain in 2 or 3 slices.
+//   64 x 64 while it makes 4 slices or more; with 2 or 3 of them the chain
+//     stays long from K = 7680, and a tile of 128 rows takes over, in the order
+//     of the measured best: three slices that fill the CUs; 4 slices (two
+//     workgroups per CU); 64 x 128; 8-wave 128 x 128 up to half the CUs' tiles.
+// Graph time over operands that no cache holds, fp16 out: the register-staged
+// split / unsplit (or 4 slices of 64 x 64 from K = 8192, where K % 512 == 0) /
+// this rule: 1 x 6144 -> 3072 13.3 / 19.2 / 10.5 us, 64 x 8320 -> 3072 18.4 /
+// 25.6 / 13.6, 154 x 7680 -> 1280 15.5 / 16.3 / 11.9, 256 x 12416 -> 3072 29.8
+// / 36.0 / 23.6, 512 x 12288 -> 3072 41.5 / 44.8 / 38.2, 512 x 15360 -> 3072
+// 48.4 / 55.2 / 45.5. On the lines, unsplit against split: 100 x 4096 -> 3072
+// 10.2 / 10.3 (2), 512 x 5120 -> 1280 12.4 / 13.1 (3), 512 x 5120 -> 3072 21.1
+// / 22.1 (2), 231 x 8192 -> 8192 33.2 / 34.4 (2), 512 x 12288 -> 5120 60.7 /
+// 69.2 (4). Over 848 shapes of up to 640 rows the rule is within 2.2% of the
+// best of all tiles and slices on average, and nowhere over 4% behind what ran
+// before it.
+static int dma_splits(int64_t M, int64_t N, int64_t K, DmaPick* tile, int* kslice) {
+  if (K < 4096) return 1;
+  const int64_t cus = device_cus();
+  const auto slices = [&](int64_t most, int64_t tiles, int64_t least) {
+    int64_t s = cus / tiles < K / least ? cus / tiles : K / least;
+    return s < most ? s : most;
+  };
+  const int64_t n64 = (N + 63) / 64, m128 = (M + 127) / 128, t64 = n64 * ((M + 63) / 64);
+  const int64_t t128 = m128 * ((N + 127) / 128);
+  const bool long_k = K >= 7680, longest_k = K >= 10240;
+  const int64_t s64 = slices(M <= 64 ? 8 : longest_k ? 6 : 4, t64, 1280);
+  const int64_t s64x128 = slices(8, n64 * m128, 1792), s128 = slices(8, t128, 1792);
+  int64_t s = 1;
+  *tile = DMA_64x64;
+  if (M <= 64 && (s64 == 2 || s64 == 3) && K / (2 * s64) >= 1280) s = 2 * s64;
+  else if (M <= 64 && s64 >= 2) s = s64;
+  else if (M <= 64 && long_k && t64 <= cus) s = 3 * t64 <= 2 * cus ? 3 : 2;
+  else if (s64 >= 4 || (!long_k && (s64 == 3 || (s64 == 2 && K >= 5120)))) s = s64;
+  else if (s64 == 3 && 10 * s64 * t64 >= 9 * cus && !longest_k) s = 3;
+  else if (s64 == 2 && long_k && !(longest_k && s64x128 >= 4 && M <= 512)) s = 4;
+  else if (s64x128 >= 3 && K >= 6144) s = s64x128, *tile = DMA_64x128;
+  else if (s128 >= 2 && long_k && 2 * t128 <= cus) s = s128, *tile = DMA_128x128D;
+  if (s < 2) return 1;
+  const int64_t slice = (K / 128 + s - 1) / s * 128;
+  *kslice = (int)slice;
+  return (int)((K + slice - 1) / slice);
 }
 
 // How a dc_w8a8_gemm call runs: the one answer that the call itself and the
@@ -1143,7 +1183,9 @@ struct RunPlan {
 static RunPlan run_plan(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, bool may_split) {
   RunPlan r{pick_dma(M, N, K, lda, ldw), 0, 1, (int)K};
   if (r.dma != DMA_NONE) {
-    if (may_split && (r.splits = dma_splits(M, N, K, &r.kslice)) > 1) r.dma = DMA_64x64;
+    DmaPick tile;
+    int kslice;
+    if (may_split && (r.splits = dma_splits(M, N, K, &tile, &kslice)) > 1) r.dma = tile, r.kslice = kslice;
     return r;
   }
   r.tile = plan_tile(M, N, K, lda, ldw);

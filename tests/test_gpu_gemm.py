@@ -234,17 +234,22 @@ def _gemm_unsplit(q, w, sx, sw, bias, dtype):
     return out
 
 
-# (M, N, K), k slices on 256 CUs: the DMA-fed kernel (K % 128 == 0), unsplit
-# and split; then the register-staged one, whose last slice is a short one
-SPLIT_K = [((512, 3072, 12288), 1), ((512, 3072, 3072), 1), ((154, 640, 4096), 1), ((77, 1280, 4096), 1),
-           ((300, 520, 8192), 4), ((154, 1280, 2048), 1), ((77, 640, 2048), 1),
-           ((154, 640, 4112), 7), ((77, 1280, 3088), 4), ((300, 520, 2112), 4), ((77, 640, 2064), 4),
-           ((512, 3072, 3088), 4)]
+# (M, N, K), and what runs it on 256 CUs: the DMA-fed kernel (K % 128 == 0)
+# unsplit, then on each tile it splits (ragged rows and columns, slices that do
+# not divide K); then the register-staged one, whose last slice is a short one
+SPLIT_K = [((512, 3072, 3072), "dma_64x128", 1), ((154, 1280, 2048), "dma_64x64", 1), ((77, 640, 2048), "dma_64x64", 1),
+           ((154, 640, 4096), "dma_64x64", 3), ((77, 1280, 4096), "dma_64x64", 3), ((300, 520, 8192), "dma_64x64", 4),
+           ((1, 5120, 7680), "dma_64x64", 6), ((33, 9000, 7808), "dma_64x64", 3), ((231, 2040, 8320), "dma_64x64", 4),
+           ((400, 640, 12416), "dma_64x128", 6), ((100, 3069, 15360), "dma_64x128", 5),
+           ((500, 1276, 6272), "dma_64x128", 3), ((512, 3072, 12288), "dma_128x128_8w", 2),
+           ((154, 3069, 7680), "dma_128x128_8w", 4),
+           ((154, 640, 4112), "128x128", 7), ((77, 1280, 3088), "128x128", 4), ((300, 520, 2112), "128x128", 4),
+           ((77, 640, 2064), "128x128", 4), ((512, 3072, 3088), "128x128", 4)]
 
 
-@pytest.mark.parametrize("mnk,slices", SPLIT_K)
+@pytest.mark.parametrize("mnk,kernel,slices", SPLIT_K)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-def test_split_k_is_bit_identical(gpu, mnk, slices, dtype):
+def test_split_k_is_bit_identical(gpu, mnk, kernel, slices, dtype):
     """Small-M, long-K problems split k over workgroups into int32 partials;
     the epilogue over their exact sum equals the unsplit GEMM and the oracle
     bit for bit. The workspace is what those slices need, no more."""
@@ -252,6 +257,7 @@ def test_split_k_is_bit_identical(gpu, mnk, slices, dtype):
     m, n, k = mnk
     ws = _lib.require().dc_w8a8_gemm_workspace_bytes(m, n, k, k, k)
     if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
+        assert _int8.gemm_kernel(m, n, k) == (kernel, slices)
         assert ws == (slices * m * n * 4 if slices > 1 else 0)
     q, w, sx, sw = _qw(m, n, k, 14)
     bias = (torch.randn(n, generator=torch.Generator().manual_seed(14)) * 0.5).to(torch.bfloat16)
@@ -525,8 +531,8 @@ def test_dma_tiles_bit_exact(gpu, mnk, kernel):
 
 @pytest.mark.parametrize("mnk", [(64, 3072, 12288), (100, 3069, 8192), (1, 16, 8704), (256, 3072, 15360)])
 def test_dma_split_k_bit_exact(gpu, mnk):
-    """Few rows over a deep K: four k slices of the DMA-fed kernel's smallest
-    tile (the workspace the library asks for) equal the unsplit call."""
+    """Few rows over a deep K: the k slices (in the workspace the library asks
+    for) equal the unsplit call."""
     m, n, k = mnk
     q, w, sx, sw = (t.to(gpu) for t in _qw(m, n, k, 17))
     bias = torch.randn(n, device=gpu).bfloat16()

@@ -321,8 +321,8 @@ def test_argument_checks_fail_before_any_launch():
     assert so.dc_w8a8_gemm(16, 32, 16, 32, 16, 16, None, 7, 16, _lib.BF16, 8, 4, 8, 32, None, 0, None) == 1
     # split-K workspace: small M with long K splits (FLUX text MLP down: 4 slices of int32 partials), big M does not
     # what the call splits into, and nothing where it runs unsplit (256 CUs)
-    assert so.dc_w8a8_gemm_workspace_bytes(64, 3072, 12288, 12288, 12288) == 4 * 64 * 3072 * 4
-    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 12288, 12288, 12288) == 0
+    assert so.dc_w8a8_gemm_workspace_bytes(64, 3072, 12288, 12288, 12288) == 5 * 64 * 3072 * 4
+    assert so.dc_w8a8_gemm_workspace_bytes(512, 3072, 12288, 12288, 12288) == 2 * 512 * 3072 * 4
     assert so.dc_w8a8_gemm_workspace_bytes(4096, 3072, 12288, 12288, 12288) == 0
     assert so.dc_w8a8_gemm_workspace_bytes(154, 1280, 2048, 2048, 2048) == 0
     assert so.dc_w8a8_gemm_workspace_bytes(154, 1280, 2064, 2064, 2064) == 4 * 154 * 1280 * 4   # 20 register-staged
@@ -498,6 +498,17 @@ def test_gemm_kernel_names_what_runs():
     for bad in ((0, 1, 16), (1, 1, 20), (1 << 31, 16, 16)):
         with pytest.raises(RuntimeError, match="no kernel takes"):
             kernel(*bad)
+
+
+@pytest.mark.parametrize("n,k", [(3072, 5120), (3072, 6144), (1280, 7680), (3072, 8320), (640, 12416), (5120, 15360)])
+def test_few_rows_over_a_deep_k_are_split(n, k):
+    """Few-row products leave no CU to a single long chain of k stages: from
+    K = 4096 they split, whatever K is modulo 512, into slices that cover the
+    CUs at most twice and of at least 1280 bytes less rounding (256 CUs)."""
+    for m in (1, 16, 64):
+        name, slices = _int8.gemm_kernel(m, n, k)
+        tiles = -(-n // 64) * -(-m // 64)
+        assert name == "dma_64x64" and 3 <= slices <= 8 and slices * tiles <= 512 and k // slices >= 1024
 
 
 def test_an_older_library_is_refused_by_its_version(monkeypatch, tmp_path):
