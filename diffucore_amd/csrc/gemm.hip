@@ -973,20 +973,6 @@ static int launch_gemm_dma(GemmArgs p, const GroupArgs& g, hipStream_t st) {
   return launch_status("w8a8_gemm_dma_kernel");
 }
 
-// Compute units of the current device (cached per device; concurrent first
-// calls store the same value).
-static int device_cus() {
-  static std::atomic<int> cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (!n) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // Tile shape by the share of the device's tile slots, over the rounds the
 // problem takes, that hold useful work (the output area M x N over all the
 // slot-tiles of those rounds, so a tile's padding past M or N counts as

@@ -235,15 +235,19 @@ static int launch_qk(QKArgs& a, int nsides, hipStream_t st) {
   return launch_status("dc_qk_norm_rope");
 }
 
-// Heads per lane group: 4 (fewer reads of the rotary matrices) while those
-// workgroups fill the chip's slots, 8 of 4 waves on each of 256 CUs; below
-// that 2, for twice the waves in flight. 24 heads of 128, q + k + v, graph
-// time over rotating buffers, 2 against 4: 512 tokens 7.8 / 8.4 us, 1024
-// 10.9 / 11.6; 3554 tokens 30.9 / 30.0, 4096 34.4 / 33.8, 8192 60.9 / 58.8.
+// Heads per lane group: 4 (fewer reads of the rotary matrices) from 3 such
+// workgroups per CU on; below that 2, for twice the waves in flight. Half
+// pairs always take 4: they read 8 matrices per lane, not 4, so what 2 heads
+// gain in waves they lose in reads. bf16, graph time over rotating buffers, 2
+// against 4 heads: adjacent pairs, D 128, q alone 8.9 / 9.1 us at 682
+// workgroups, 11.3 / 11.1 at 900, 16.4 / 15.9 at 1536; q + k 8.9 / 9.1 at 768,
+// 12.8 / 12.4 at 1152; D 64, q alone 8.2 / 8.8 at 640, 13.7 / 13.6 at 1280;
+// half pairs, q + k 5.8 / 5.6 at 192, 12.6 / 10.9 at 768, 34.7 / 28.6 at 3072.
 template <int DT, int LPR>
 static int launch_qk_heads(QKArgs& a, int nsides, hipStream_t st) {
-  constexpr int64_t SLOT_ROWS = 8 * 256 * (int64_t)(256 / LPR) * 4;   // rows those slots hold, 4 per lane group
-  if (a.H % 4 == 0 && (int64_t)a.rows * nsides >= SLOT_ROWS) return launch_qk<DT, LPR, 4>(a, nsides, st);
+  const int64_t wg4 = (int64_t)a.rows * nsides / (256 / LPR * 4);   // workgroups at 4 heads per lane group
+  const bool four = (a.flags & DC_QK_ROPE_HALF) || wg4 >= 3 * (int64_t)device_cus();
+  if (a.H % 4 == 0 && four) return launch_qk<DT, LPR, 4>(a, nsides, st);
   if (a.H % 2 == 0) return launch_qk<DT, LPR, 2>(a, nsides, st);
   return launch_qk<DT, LPR, 1>(a, nsides, st);
 }

@@ -171,13 +171,17 @@ def test_rejects_what_it_cannot_take(gpu):
 
 @pytest.mark.parametrize("B,L,H,D", [
     (1, 1, 24, 128), (1, 3, 4, 64),                                         # less than one turn of 8 workgroups
-    (1, 1820, 24, 128), (1, 1821, 24, 128), (2, 911, 24, 128),              # either side of the 2 / 4 heads line
+    (1, 1820, 24, 128), (1, 1821, 24, 128), (2, 911, 24, 128),
+    (1, 682, 24, 128), (1, 683, 24, 128), (1, 1023, 24, 128), (2, 512, 24, 128),   # either side of the 2 / 4 heads
+    (1, 2047, 24, 128), (1, 2048, 24, 128),                                        # line for 3, 2 and 1 sides
     (1, 43, 6, 128), (1, 129, 1, 128), (3, 1025, 2, 32), (1, 517, 7, 256)])
 @pytest.mark.parametrize("sides", [1, 2, 3])
-def test_sides_in_turns(gpu, B, L, H, D, sides):
+@pytest.mark.parametrize("half", [False, True])
+def test_sides_in_turns(gpu, B, L, H, D, sides, half):
     """q alone, q and k, or q, k and v of a stacked projection in one launch:
     each output is that of its own launch bit for bit, v's a plain copy, and
-    nothing past the last row is written."""
+    nothing past the last row is written; with both pairings of the rotary
+    embedding."""
     g = torch.Generator(device=gpu).manual_seed(L + H)
     x = torch.randn(B, L, 3, H, D, device=gpu, generator=g).bfloat16()
     wq, wk = ((torch.rand(D, device=gpu, generator=g) + 0.5).bfloat16() for _ in range(2))
@@ -185,15 +189,21 @@ def test_sides_in_turns(gpu, B, L, H, D, sides):
     bufs = [torch.full((B + 1, L, H, D), 7.0, device=gpu, dtype=torch.bfloat16) for _ in range(3)]
     oq, ok, ov = (b[:B] for b in bufs)
     q, k, v = x[:, :, 0], x[:, :, 1], x[:, :, 2]
-    kw = {}
+    kw = dict(half_pairs=half)
     if sides > 1:
         kw.update(k=k, k_weight=wk, out_k=ok)
     if sides > 2:
         kw.update(v=v, out_v=ov)
     QK.norm_rope(q, wq, 1e-6, pe, out_q=oq, **kw)
-    _close(oq, _eager_flux(q, wq, pe), torch.bfloat16)
+    if half:   # the half pairs (i, i + D/2) are the adjacent ones of interleaved channels
+        inter = torch.arange(D, device=gpu).view(2, D // 2).t().reshape(-1)
+        want = torch.empty_like(oq)
+        want[..., inter] = _eager_flux(q[..., inter], wq[inter], pe)
+    else:
+        want = _eager_flux(q, wq, pe)
+    _close(oq, want, torch.bfloat16)
     if sides > 1:
-        assert torch.equal(ok, QK.norm_rope(k, wk, 1e-6, pe)[0])
+        assert torch.equal(ok, QK.norm_rope(k, wk, 1e-6, pe, half_pairs=half)[0])
     if sides > 2:
         assert torch.equal(ov, v)
     for b in bufs[:sides]:
