@@ -19,15 +19,20 @@
 // for all of them, and each lane issues all its loads before any arithmetic.
 // A workgroup of 256 threads takes 256/(D/8) lane groups. q, k and an
 // optional plain copy of v (to gather two
-// streams' v into one buffer for the attention) run in one launch, taking
-// turns 8 workgroups at a time. The kernel is bound by HBM: 2 bytes read and
-// 2 written per element, the weights and the frequency rows come from cache.
-// With one contiguous range of workgroups each for q, k and v instead, the
-// three passes over a stacked [.., 3, H, D] projection each skipped two thirds
-// of every row and read the frequency rows from HBM again: 4096 tokens x 24
-// heads x 128 bf16 38.6 -> 32.9 us (155 MB, 4.7 TB/s), 2 x 4096 67.1 -> 57.5,
-// 2 x 1777 33.0 -> 29.2 (graph time over rotating buffers; separate q / k / v
-// buffers 37.0 -> 33.1 at 4096).
+// streams' v into one buffer for the attention) run in one launch. The kernel
+// is bound by HBM: 2 bytes read and 2 written per element, the weights and the
+// frequency rows come from cache.
+// Order of the workgroups: q, k and v take turns 8 at a time from 8 workgroups
+// (of 4 heads per lane group) per CU on, else each is one contiguous range.
+// Past what the chip holds at once, three ranges over a stacked [.., 3, H, D]
+// projection each skip two thirds of every row and read the frequency rows
+// from HBM again: 24 heads x 128 bf16, ranges against turns, 8192 tokens 68.3 /
+// 59.0 us, 4096 35.3 / 31.1 (155 MB, 5.0 TB/s), 3000 29.2 / 26.3, 2400 24.5 /
+// 22.1, 1820 18.4 / 18.3. Below, all of it runs at once, and turns put the
+// cheap copies of v between the others: 1024 tokens 12.3 / 12.7, 512 7.0 / 7.4,
+// 256 5.3 / 5.5, half pairs at 256 6.5 / 7.8. With q and k only neither order
+// skips much: 4096 tokens 26.2 / 26.2, 1024 8.9 / 9.0 (graph time over rotating
+// buffers).
 #include "common.h"
 
 namespace dc {
@@ -46,6 +51,7 @@ struct QKArgs {
   int L, H;
   int rows;            // B * L * H
   int nsides;          // 1 (q), 2 (and k or v) or 3
+  int range;           // workgroups of one side, each a contiguous range; 0: the sides take turns
   int flags;           // DC_QK_* bits
   int w_f32;           // weights are float32 (else the activation dtype)
   float eps, inv_d;
@@ -120,12 +126,19 @@ __device__ __forceinline__ float partner(float v) {
 template <int DT, int LPR, int NH>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(QKArgs a) {
   constexpr int RPW = 256 / LPR;   // lane groups per workgroup
-  // q, k and v take turns 8 workgroups at a time (launch_qk pads each to a
-  // multiple of 8): workgroups go round-robin over 8 XCDs, so a token's q, k
-  // and v run close together in time and on one XCD
-  const int turn = blockIdx.x >> 3;
-  const int side = turn % a.nsides;
-  const unsigned blk = (unsigned)(turn / a.nsides) * 8u + (blockIdx.x & 7u);
+  int side;
+  unsigned blk;
+  if (a.range) {
+    side = blockIdx.x / a.range;
+    blk = blockIdx.x - side * a.range;
+  } else {
+    // turns of 8 workgroups (launch_qk pads each side to a multiple of 8):
+    // workgroups go round-robin over 8 XCDs, so a token's q, k and v run close
+    // together in time and on one XCD
+    const int turn = blockIdx.x >> 3;
+    side = turn % a.nsides;
+    blk = (unsigned)(turn / a.nsides) * 8u + (blockIdx.x & 7u);
+  }
   const unsigned ugrp = blk * RPW + threadIdx.x / LPR;   // rows NH * grp .. NH * grp + NH - 1
   const int j = (int)threadIdx.x % LPR;
   if (ugrp >= (unsigned)a.rows / NH) return;  // whole groups leave together: the lane exchanges stay inside live rows
@@ -226,11 +239,13 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(QKArgs a) {
 }
 
 template <int DT, int LPR, int NH>
-static int launch_qk(QKArgs& a, int nsides, hipStream_t st) {
+static int launch_qk(QKArgs& a, int nsides, bool turns, hipStream_t st) {
   constexpr int RPW = 256 / LPR;
   const int groups = a.rows / NH;   // H % NH == 0, so rows % NH == 0
-  const unsigned blocks = (unsigned)((groups + RPW - 1) / RPW + 7) / 8 * 8;   // of one side
+  unsigned blocks = (unsigned)((groups + RPW - 1) / RPW);   // of one side
+  if (turns) blocks = (blocks + 7) / 8 * 8;
   a.nsides = nsides;
+  a.range = turns ? 0 : (int)blocks;
   hipLaunchKernelGGL((qk_norm_rope_kernel<DT, LPR, NH>), dim3(blocks * nsides), dim3(256), 0, st, a);
   return launch_status("dc_qk_norm_rope");
 }
@@ -247,9 +262,10 @@ template <int DT, int LPR>
 static int launch_qk_heads(QKArgs& a, int nsides, hipStream_t st) {
   const int64_t wg4 = (int64_t)a.rows * nsides / (256 / LPR * 4);   // workgroups at 4 heads per lane group
   const bool four = (a.flags & DC_QK_ROPE_HALF) || wg4 >= 3 * (int64_t)device_cus();
-  if (a.H % 4 == 0 && four) return launch_qk<DT, LPR, 4>(a, nsides, st);
-  if (a.H % 2 == 0) return launch_qk<DT, LPR, 2>(a, nsides, st);
-  return launch_qk<DT, LPR, 1>(a, nsides, st);
+  const bool turns = nsides == 3 && wg4 >= 8 * (int64_t)device_cus();
+  if (a.H % 4 == 0 && four) return launch_qk<DT, LPR, 4>(a, nsides, turns, st);
+  if (a.H % 2 == 0) return launch_qk<DT, LPR, 2>(a, nsides, turns, st);
+  return launch_qk<DT, LPR, 1>(a, nsides, turns, st);
 }
 
 template <int DT>

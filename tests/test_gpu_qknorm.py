@@ -170,8 +170,9 @@ def test_rejects_what_it_cannot_take(gpu):
 
 
 @pytest.mark.parametrize("B,L,H,D", [
-    (1, 1, 24, 128), (1, 3, 4, 64),                                         # less than one turn of 8 workgroups
-    (1, 1820, 24, 128), (1, 1821, 24, 128), (2, 911, 24, 128),
+    (1, 1, 24, 128), (1, 3, 4, 64),
+    (1, 1820, 24, 128), (1, 1821, 24, 128), (2, 911, 24, 128),              # either side of the line for turns
+    (1, 7291, 6, 128), (1, 43700, 1, 128), (1, 5462, 4, 256),               # turns with 2, 1 and 4 heads, ragged ends
     (1, 682, 24, 128), (1, 683, 24, 128), (1, 1023, 24, 128), (2, 512, 24, 128),   # either side of the 2 / 4 heads
     (1, 2047, 24, 128), (1, 2048, 24, 128),                                        # line for 3, 2 and 1 sides
     (1, 43, 6, 128), (1, 129, 1, 128), (3, 1025, 2, 32), (1, 517, 7, 256)])
