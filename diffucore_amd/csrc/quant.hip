@@ -379,6 +379,9 @@ __device__ __forceinline__ float gelu_erf_f32(float x) {
   p = __builtin_fmaf(p, t, 1.00002368f * LOG2E);
   p = __builtin_fmaf(p, t, -1.26551223f * LOG2E - 1.0f);
   const float h = t * __builtin_amdgcn_exp2f(__builtin_fmaf(x * x, -0.5f * LOG2E, p));
+  // the float's sign, not the 16-bit input's: comparing that would keep the
+  // packed inputs live to the end (fp16: 58 VGPRs, 8 waves per SIMD; 68 and 7)
+  x = materialize(x);
   return x * (x < 0.0f ? h : 1.0f - h);
 }
 
@@ -387,17 +390,26 @@ __device__ __forceinline__ float act_f32(float x) {
   return ACT == DC_ACT_GELU_TANH ? gelu_tanh_f32(x) : gelu_erf_f32(x);
 }
 
-// Two floats rounded to DT and back; bf16 pairs in one conversion
-template <int DT>
+// Two floats rounded to DT and back, 16-bit pairs in one conversion. fp16
+// values pass materialize first: the compiler otherwise folds the product that
+// made them into the conversion (v_fma_mixlo_f16), which rounds once, to fp16,
+// where the GELU is rounded to float32 and then to fp16. PK16 = false converts
+// fp16 one by one: GEGLU at 4096 x 12288 takes 66 us so and 76 packed.
+template <int DT, bool PK16 = true>
 __device__ __forceinline__ void round_pair(float& a, float& b) {
   if constexpr (DT == DC_BF16) {
     const v2f x = {a, b};
     const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
     a = __uint_as_float(u << 16);
     b = __uint_as_float(u & 0xffff0000u);
+  } else if constexpr (DT == DC_F16 && PK16) {
+    const v2f x = {materialize(a), materialize(b)};
+    const v2h h = __builtin_convertvector(x, v2h);
+    a = (float)h[0];
+    b = (float)h[1];
   } else {
-    a = round_to<DT>(a);
-    b = round_to<DT>(b);
+    a = round_to<DT>(materialize(a));
+    b = round_to<DT>(materialize(b));
   }
 }
 
@@ -411,7 +423,8 @@ __device__ __forceinline__ void round_pair(float& a, float& b) {
 // per element, the GELU's constants folded and bf16 rounded in pairs (28.5
 // an element before), 512 x 12288 tanh 11.8 -> 10.8 us, 4608 x (3072 + 12288)
 // 62.4 -> 59.4, 4096 x 8192 erf 42.0 -> 39.4 (graph time over rotating
-// buffers); 4096 x 12288 51.1 -> 48.9; GEGLU 2048 x 10240 level at 20.
+// buffers); 4096 x 12288 51.1 -> 48.9; GEGLU 2048 x 10240 level at 20. fp16:
+// 4096 x 12288 erf 61.4 -> 58.9, tanh 48.7 -> 47.9, 4096 x 8192 erf 42.2 -> 40.4.
 template <int DT, int S, bool ROT, int ACT>
 __global__ void __launch_bounds__(1024) quant_act_rows_kernel(const void* __restrict__ x1, int64_t ld1, int K1,
                                                               const void* __restrict__ x2, int64_t ld2, int K, int64_t M,
@@ -449,10 +462,15 @@ __global__ void __launch_bounds__(1024) quant_act_rows_kernel(const void* __rest
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
           float g0 = act_f32<DC_ACT_GELU_ERF>(gt[0][j][e]), g1 = act_f32<DC_ACT_GELU_ERF>(gt[0][j][e + 1]);
-          round_pair<DT>(g0, g1);
-          v[0][j][e] *= g0;
-          v[0][j][e + 1] *= g1;
-          round_pair<DT>(v[0][j][e], v[0][j][e + 1]);
+          round_pair<DT, false>(g0, g1);
+          if constexpr (DT == DC_F16) {   // the product of two fp16 values is exact: folding it changes nothing
+            v[0][j][e] = round_to<DT>(v[0][j][e] * g0);
+            v[0][j][e + 1] = round_to<DT>(v[0][j][e + 1] * g1);
+          } else {
+            v[0][j][e] *= g0;
+            v[0][j][e + 1] *= g1;
+            round_pair<DT>(v[0][j][e], v[0][j][e + 1]);
+          }
         }
     }
   }

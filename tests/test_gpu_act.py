@@ -236,3 +236,16 @@ def test_int8_geglu_ff_matches_eager(gpu, dim, bias):
     af, gf = proj(x).chunk(2, dim=-1)
     y_float = out(af * F.gelu(gf))
     assert rel_l2(np32(y), np32(y_float)) < 3e-2 and cosine(np32(y), np32(y_float)) > 0.999
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("group", [0, 256])
+def test_geglu_of_ones_is_gelu(gpu, dtype, group):
+    """Every finite 16-bit value through GEGLU with a value half of ones (the
+    product is exact) gives the codes and scales of the GELU alone: both forms
+    round it to float32 and then to the dtype, whichever way they convert."""
+    x = torch.arange(1 << 16, dtype=torch.int32, device=gpu).to(torch.int16).view(dtype)
+    x = torch.where(x.isfinite(), x, torch.zeros_like(x)).view(-1, 256)
+    q, s = _int8.act_quantize(x, group, "gelu")
+    qg, sg = _int8.act_quantize(torch.cat((torch.ones_like(x), x), 1), group, "geglu")
+    assert torch.equal(q, qg) and torch.equal(s, sg)
