@@ -125,7 +125,7 @@ for i, (rc, want) in enumerate(checks):
         sys.exit(3)
     if rc:
         assert last(), i
-assert gws(512, 3072, 12288, 12288, 12288) == 4 * 512 * 3072 * 4
+assert gws(512, 3072, 12288, 12288, 12288) == 2 * 512 * 3072 * 4   # two k slices (256 CUs)
 assert aws(1, 1, 1, 1, 200) == 0
 print("asan child ok", len(checks))
 '''
