@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime first)
 LIB_PATH = Path(__file__).resolve().parent / "libdiffucore_amd.so"
 
 F16, BF16, F32, I32, NONE = 0, 1, 2, 3, -1
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _DTYPE = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32, torch.int32: I32}
 
@@ -38,6 +38,7 @@ _SIGS = {
     "dc_w8a8_gemm_grouped": (_I, [_P, _I, _I64, _I64, _I, _I, _P]),
     "dc_w8a8_gemm_grouped_gated": (_I, [_P, _P, _I, _I64, _I64, _I, _I, _P]),
     "dc_w8a8_gemm_group_plan": (_I, [ctypes.POINTER(_I64), _I, _I64, _I64]),
+    "dc_w8a8_gemm_gated_plan": (_I, [ctypes.POINTER(_I64), _I, _I64, _I64]),
     "dc_rescale": (_I, [_P, _I64, _P, _P, _P, _I, _P, _I, _I64, _I64, _I64, _P]),
     "dc_ln_mod_quantize_rows": (_I, [_P, _I, _I64, _I64, _I64, _P, _P, _I, _I64, _I64, ctypes.c_float, _I, _P, _I64, _P, _P]),
     "dc_act_quantize_rows": (_I, [_P, _I64, _I64, _P, _I64, _I64, _I, _I, _I64, _I, _P, _I64, _P, _P]),

@@ -1388,28 +1388,59 @@ static int group_bias(GemmArgs p, const GroupArgs& g, int bias_dtype, hipStream_
 
 static int64_t dma_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256); }
 
-extern "C" int dc_w8a8_gemm_group_plan(const int64_t* Ms, int count, int64_t N, int64_t K) {
+// Whether a grouped launch pays. It runs 256 x 256 tiles, one per CU, where
+// separate calls take whichever tiles suit each problem: so only where its
+// tiles need no more rounds of the CUs than the largest problem's alone, and
+//   plain  its one round holds at least 9/16 of the CUs' worth of outputs, or
+//          the last of several at least 2/5 of their tiles;
+//   gated  (each separate call is followed by two torch passes) its one round
+//          holds K / 64 tiles' worth, at most 3/8 of the CUs'.
+// bf16, graph time, separate / grouped us. Plain: 512 + 512 rows x 3072 ->
+// 3072 (48 tiles) 22.9 / 35.8, 1536 + 512 (96) 37.8 / 38.2, 2816 + 512 (156) 48.0 /
+// 42.6, 4096 + 512 (216) 56.3 / 48.6, 512 + 512 x 3072 -> 9216 (144) 65.6 /
+// 47.2, x 12288 -> 3072 256 + 256 (24) 52.1 / 153.3, 2048 + 512 (120) 145 / 150,
+// 4096 + 512 184.8 / 163.3; 6144 + 512 x 3072 -> 3072 (256 + 56) 86.7 / 93.5,
+// 2048 + 512 x 3072 -> 9216 (256 + 104) 117.5 / 96.2, 3600 + 256 (512 + 64)
+// 135.6 / 148.7, 4096 + 512 (512 + 136) 157.5 / 149.6. Gated: 256 + 256 x 3072 ->
+// 3072 32.0 / 38.6, 512 + 512 (48) 40.1 / 38.8, 512 + 512 x 1280 -> 1280 (20) 24.8 /
+// 23.4, 2048 + 2048 x 5120 -> 1280 (80) 66.4 / 59.1, 1024 + 512 x 12288 -> 3072
+// (72) 119 / 149, 1536 + 512 (96) 149 / 148.
+static int group_plan(const char* who, const int64_t* Ms, int count, int64_t N, int64_t K, bool gated) {
   clear_error();
   if (!Ms || count < 1 || count > DC_GEMM_MAX_GROUP || N <= 0 || K <= 0) {
-    set_error("dc_w8a8_gemm_group_plan: bad arguments");
+    set_error("%s: bad arguments", who);
     return -1;
   }
   int live = 0;
   int64_t total = 0, largest = 0;
+  double rows = 0.0;
   for (int i = 0; i < count; ++i) {
     if (Ms[i] < 0) {
-      set_error("dc_w8a8_gemm_group_plan: negative M");
+      set_error("%s: negative M", who);
       return -1;
     }
     if (Ms[i] == 0) continue;
     ++live;
     const int64_t t = dma_tiles(Ms[i], N);
     total += t;
+    rows += (double)Ms[i];
     largest = t > largest ? t : largest;
   }
   if (K % 256 || live < 2) return 0;
   const int64_t cus = device_cus();
-  return (total + cus - 1) / cus <= (largest + cus - 1) / cus ? 1 : 0;
+  if ((total + cus - 1) / cus > (largest + cus - 1) / cus) return 0;
+  const double worth = rows * (double)N / (256.0 * 256.0);   // in tiles
+  const int64_t last = (total - 1) % cus + 1;                // tiles of the last round
+  if (gated) return total > cus || worth >= (double)(K / 64 < 3 * cus / 8 ? K / 64 : 3 * cus / 8);
+  return total > cus ? 5 * last >= 2 * cus : 16.0 * worth >= 9.0 * (double)cus;
+}
+
+extern "C" int dc_w8a8_gemm_group_plan(const int64_t* Ms, int count, int64_t N, int64_t K) {
+  return group_plan("dc_w8a8_gemm_group_plan", Ms, count, N, K, false);
+}
+
+extern "C" int dc_w8a8_gemm_gated_plan(const int64_t* Ms, int count, int64_t N, int64_t K) {
+  return group_plan("dc_w8a8_gemm_gated_plan", Ms, count, N, K, true);
 }
 
 static int group_fail(int code, const char* who, const char* msg) {

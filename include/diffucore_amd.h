@@ -273,13 +273,16 @@ int dc_w8a8_gemm_grouped_gated(const dc_gemm_problem* problems, const dc_gemm_ga
 
 /*
  * Whether one dc_w8a8_gemm_grouped launch over problems of these row counts
- * is expected to beat separate dc_w8a8_gemm calls on the current device: 1
- * when K % 256 == 0, there are at least two non-empty problems and their
- * 256 x 256 tiles together need no more rounds of the device's CUs than the
- * largest problem's alone; 0 otherwise; -1 for bad arguments. No counterpart
- * in the reference.
+ * (group_plan), or one dc_w8a8_gemm_grouped_gated launch (gated_plan, against
+ * calls each followed by the two elementwise passes), is expected to beat
+ * separate dc_w8a8_gemm calls on the current device: 1 only when K % 256 == 0,
+ * there are at least two non-empty problems, their 256 x 256 tiles together
+ * need no more rounds of the device's CUs than the largest problem's alone,
+ * and those rounds are full enough (measured lines); 0 otherwise; -1 for bad
+ * arguments. No counterpart in the reference.
  */
 int dc_w8a8_gemm_group_plan(const int64_t* Ms, int count, int64_t N, int64_t K);
+int dc_w8a8_gemm_gated_plan(const int64_t* Ms, int count, int64_t N, int64_t K);
 
 /*
  * The rescale pass on an int32 accumulator, for callers that hold one.

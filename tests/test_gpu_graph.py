@@ -5,10 +5,11 @@ synchronizations, the outputs are overwritten with NaN before each replay
 (so a replay that skips a write shows), and new values written into the
 captured input buffers must reach the next replay.
 
-Covered: the quantize kernel, each GEMM plan the FLUX step uses (DMA-fed
-256 x 256, 192 x 128 at the text MLP-up shape, 192 x 256 / 128 x 128,
-split-K with its workspace and epilogue pass, a grouped launch of two
-layers, the same pair with the gated residual epilogue) and the INT8 attention (K statistics, K quantize, attention): the
+Covered: the quantize kernel, GEMM tiles of the FLUX step (DMA-fed 128 x 128
+and 64 x 128, register-staged 192 x 128 at the text MLP-up shape),
+split-K with its workspace and epilogue pass, a grouped launch of two layers
+on 256 x 256 tiles, the same pair with the gated residual epilogue, and the
+INT8 attention (K statistics, K quantize, attention): the
 DMA-fed kernel with 256-query tiles at the FLUX shape, with 128-query tiles
 and stream-K pieces plus their merge at SDXL's 4096-token self-attention and
 with whole 128-query tiles at head dim 64, and the register-staged 128-query
@@ -27,11 +28,12 @@ from diffucore_amd import _int8, attention_bhld
 pytestmark = pytest.mark.gpu
 
 BF16 = torch.bfloat16
-# (M, K, N): DMA-fed 256 x 256 plan, split-K (M = 512, K = 3072), 192 x 128
-# tiles (FLUX's text MLP up), a ragged one; the last two run as one grouped
-# launch (dc_w8a8_gemm_grouped)
-LINEARS = [(4096, 512, 4096), (512, 3072, 3072), (512, 3072, 12288), (1000, 768, 1280), (1024, 512, 1024),
-           (300, 512, 1024)]
+# (M, K, N): 256 x 256 class, 64 x 128 tiles, the register-staged 192 x 128
+# (FLUX's text MLP up), a ragged one, split-K on the DMA-fed and the
+# register-staged kernel; the last two run as one grouped launch
+# (dc_w8a8_gemm_grouped)
+LINEARS = [(4096, 512, 4096), (512, 3072, 3072), (512, 3072, 12288), (1000, 768, 1280), (512, 12288, 1024),
+           (154, 4112, 640), (2304, 512, 4096), (300, 512, 4096)]
 NS = len(LINEARS) - 2   # the layers called one by one
 ATTN = [(1, 24, 4608, 128), (2, 10, 4096, 64), (1, 4, 1000, 64), (1, 4, 4096, 128)]
 
@@ -39,7 +41,8 @@ ATTN = [(1, 24, 4608, 128), (2, 10, 4096, 64), (1, 4, 1000, 64), (1, 4, 4096, 12
 def _case(gpu, seed):
     g = torch.Generator(device=gpu).manual_seed(seed)
     torch.manual_seed(seed)
-    layers = [_int8.Int8Linear.from_linear(nn.Linear(k, n, bias=True).to(gpu).to(BF16), 256) for _, k, n in LINEARS]
+    layers = [_int8.Int8Linear.from_linear(nn.Linear(k, n, bias=True).to(gpu).to(BF16), 256 if k % 256 == 0 else 0)
+              for _, k, n in LINEARS]
     xs = [torch.randn(m, k, generator=g, device=gpu).to(BF16) for m, k, _ in LINEARS]
     # residuals and one-row gates for the gated pair (the last two layers)
     xs += [torch.randn(m, n, generator=g, device=gpu).to(BF16) for m, _, n in LINEARS[NS:]]
@@ -63,6 +66,7 @@ def test_graph_replays_equal_eager_calls(gpu):
     m, k, n = LINEARS[0]
     assert _int8.gemm_plan(m, n, k) == "dma_256x256"
     if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
+        assert _int8.gemm_kernel(512, 1024, 12288)[1] > 1 and _int8.gemm_kernel(154, 640, 4112) == ("128x128", 7)
         assert _int8.gemm_plan(LINEARS[2][0], LINEARS[2][2], LINEARS[2][1]) == "192x128"
         assert _int8.gemm_kernel(LINEARS[2][0], LINEARS[2][2], LINEARS[2][1]) == ("192x128", 1)
     assert _int8.gemm_group_plan([LINEARS[NS][0], LINEARS[NS + 1][0]], LINEARS[NS][2], LINEARS[NS][1])

@@ -412,6 +412,21 @@ def test_argument_checks_fail_before_any_launch():
     assert so.dc_w8a8_gemm_group_plan(Ms, 2, 3072, 3000) == 0          # K not a multiple of 256
     assert so.dc_w8a8_gemm_group_plan(Ms, 1, 3072, 3072) == 0          # one problem
     assert so.dc_w8a8_gemm_group_plan(Ms, 0, 3072, 3072) == -1
+    assert so.dc_w8a8_gemm_gated_plan(Ms, 0, 3072, 3072) == -1 and b"gated_plan" in so.dc_last_error()
+    # measured against the separate calls: a launch that leaves most CUs idle,
+    # or a nearly empty last round, loses to them (M, M, N, K, plain, gated)
+    for m1, m2, n, k, plain, gate in ((256, 256, 3072, 12288, 0, 0), (64, 64, 9216, 3072, 0, 0),
+                                      (512, 512, 3072, 3072, 0, 1), (1024, 512, 3072, 3072, 0, 1),
+                                      (2816, 512, 3072, 3072, 1, 1), (512, 512, 9216, 3072, 1, 1),
+                                      (1024, 512, 3072, 12288, 0, 0), (1536, 512, 3072, 12288, 0, 1),
+                                      (512, 512, 1280, 1280, 0, 1), (3072, 512, 1280, 5120, 0, 0),
+                                      (6144, 512, 3072, 3072, 0, 1), (2048, 512, 9216, 3072, 1, 1),
+                                      (3600, 256, 9216, 3072, 0, 1), (4096, 512, 9216, 3072, 1, 1),
+                                      (4096, 512, 12288, 3072, 0, 0)):
+        pair = (_lib.ctypes.c_int64 * 2)(m1, m2)
+        assert (so.dc_w8a8_gemm_group_plan(pair, 2, n, k), so.dc_w8a8_gemm_gated_plan(pair, 2, n, k)) == (plain, gate)
+        assert _int8.gemm_group_plan([m1, m2], n, k) == bool(plain)
+        assert _int8.gemm_group_plan([m1, m2], n, k, gated=True) == bool(gate)
 
 
 def test_bench_cpu_configs_reports_every_shape(monkeypatch, capsys):
