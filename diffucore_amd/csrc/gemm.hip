@@ -1038,15 +1038,11 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
 //     (29.2).
 //   t128 <= 2 CUs: two 4-wave 128 x 128 workgroups per CU, one's epilogue
 //     under the other's products: 2048 x 1280 -> 3840 17.4 -> 14.2 (256 x 256:
-//     18.9), 8192 x 2560 -> 640 26.8 -> 19.8 (29.7). Where they leave some CUs
-//     with two and some with one while the register-staged 192 x 128 tile
-//     gives each CU at most one (its class), that tile stays from K > 2048 on
-//     4 to 8 m tiles: 512 x 3072 -> 12288 32.0 (two 128 x 128: 33.7), 512 x
-//     6144 -> 9216 53.8 (59.8), 640 x 2560 -> 7680 26.7 (30.4), 1024 x 12288 ->
-//     6144 101.2 (114.5). Level at K = 2048 (22.2 against 21.9 at 512 rows,
-//     22.5 against 22.3 at 1024) and past the rows (2048 x 3072 -> 3072 29.9
-//     against 30.8, 2048 x 4096 -> 3072 37.3 against 36.0; 4096 x 4096 -> 1536
-//     37.7 against 34.6; 300 x 4096 -> 13000 39.8 against 37.6).
+//     18.9), 8192 x 2560 -> 640 26.8 -> 19.8 (29.7). Against one register-
+//     staged 192 x 128 tile per CU the two take 2 to 9% longer with the operands
+//     in HBM and up to 24% less with them in the Infinity Cache: 512 x 3072 ->
+//     12288 33.8 and 26.1 (32.8 and 32.5), 512 x 6144 -> 9216 59.5 and 39.5
+//     (54.8 and 51.5), 1024 x 12288 -> 6144 113.1 and 80.7 (104.3 and 105.4).
 //   above: the least time by a fit of the measured times, a fixed part and a
 //     part per round of the device's slots, linear in K. A last round of
 //     128 x 128 tiles that puts one on each CU takes 0.65 of a full one; the
@@ -1076,11 +1072,7 @@ static DmaPick pick_dma(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
   const int64_t t128 = tiles(128, 128);
   if (t128 <= cus / 2) return tiles(64, 128) < cus / 2 ? DMA_64x64 : DMA_64x128;
   if (t128 <= cus) return DMA_128x128D;
-  if (t128 <= 2 * cus) {
-    const int64_t m128 = (M + 127) / 128;
-    return K > 2048 && m128 >= 4 && m128 <= 8 && plan_tile(M, N, K, lda, ldw) == DC_GEMM_PLAN_192x128 ? DMA_NONE
-                                                                                                      : DMA_128x128;
-  }
+  if (t128 <= 2 * cus) return DMA_128x128;
   const double k = (double)K;
   const auto rounds = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
   const int64_t full = t128 / (2 * cus), rest = t128 % (2 * cus);

@@ -68,7 +68,7 @@ def test_graph_replays_equal_eager_calls(gpu):
     if torch.cuda.get_device_properties(gpu).multi_processor_count == 256:
         assert _int8.gemm_kernel(512, 1024, 12288)[1] > 1 and _int8.gemm_kernel(154, 640, 4112) == ("128x128", 7)
         assert _int8.gemm_plan(LINEARS[2][0], LINEARS[2][2], LINEARS[2][1]) == "192x128"
-        assert _int8.gemm_kernel(LINEARS[2][0], LINEARS[2][2], LINEARS[2][1]) == ("192x128", 1)
+        assert _int8.gemm_kernel(LINEARS[2][0], LINEARS[2][2], LINEARS[2][1]) == ("dma_128x128", 1)
     assert _int8.gemm_group_plan([LINEARS[NS][0], LINEARS[NS + 1][0]], LINEARS[NS][2], LINEARS[NS][1])
     assert all(x.data_ptr() % 16 == 0 for x in xs[NS + 2:])   # the gated pair takes the fused epilogue
     with torch.no_grad():

@@ -498,9 +498,7 @@ def test_gemm_kernel_names_what_runs():
     kernel = _int8.gemm_kernel
     assert kernel(4608, 21504, 3072) == ("dma_256x256", 1)      # linear1
     assert kernel(4096, 9216, 3072) == ("dma_192x256", 1)       # image qkv
-    assert kernel(512, 12288, 3072) == ("192x128", 1)           # text MLP up: one register-staged tile per CU
-    assert kernel(512, 12288, 2048) == ("dma_128x128", 1)       # up to K = 2048 two DMA-fed ones are level
-    assert kernel(2048, 3840, 3072) == ("dma_128x128", 1)
+    assert kernel(512, 12288, 3072) == ("dma_128x128", 1)       # text MLP up: class 192x128
     assert kernel(2048, 1280, 1280) == ("dma_128x128_8w", 1)
     assert kernel(512, 3072, 3072) == ("dma_64x128", 1)
     assert kernel(154, 2560, 2048) == ("dma_64x64", 1)
