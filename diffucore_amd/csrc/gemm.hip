@@ -993,8 +993,9 @@ static int launch_gemm_dma(GemmArgs p, const GroupArgs& g, hipStream_t st) {
 // smaller one finishes first) and pad N by at most 2% (SDXL's N = 640 pads
 // to 768: 128 x 128 tiles measured 7% faster there, 11.1 against 11.9 us at
 // 8192 x 640 -> 640). Measured: FLUX's 512-row text MLP up 33.2 -> 30.5 us
-// and qkv 31.6 -> 27.8 us; the choice is unchanged on the other SD1.5 /
-// SDXL / FLUX shapes.
+// and qkv 31.6 -> 27.8 us. All of these figures are of the register-staged
+// kernel, when it ran every shape; of the shapes named it still runs the
+// text stream's.
 // Tile class of a problem: DC_GEMM_PLAN_* (dc_w8a8_gemm_plan; run_plan takes it for
 // the register-staged kernel where pick_dma has no tile).
 static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
@@ -1031,7 +1032,7 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
 //     bounds these) over more CUs. 64 x 64 while 64 x 128 tiles would fill
 //     under half the CUs: 154 x 2048 -> 2560 14.4 -> 6.2 us (64 x 128: 7.2;
 //     128 x 128: 9.8); else 64 x 128: 512 x 3072 -> 3072 21.5 -> 10.7 (64 x 64:
-//     11.9), 512 x 12288 -> 3072 38.8 -> 30.9 (36.5; 128 x 128: 40).
+//     11.9). Deep K on few rows is then split (dma_splits).
 //   t128 <= CUs: one 8-wave 128 x 128 tile per CU, two waves per SIMD and 3
 //     stages to hide the loads no other workgroup hides: 2048 x 1280 -> 1280
 //     11.3 -> 8.6 (4 waves, two stages: 10.4), 2048 x 5120 -> 1280 30.3 -> 21.2
@@ -1043,17 +1044,22 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) 
 //     in HBM and up to 24% less with them in the Infinity Cache: 512 x 3072 ->
 //     12288 33.8 and 26.1 (32.8 and 32.5), 512 x 6144 -> 9216 59.5 and 39.5
 //     (54.8 and 51.5), 1024 x 12288 -> 6144 113.1 and 80.7 (104.3 and 105.4).
-//   above: the least time by a fit of the measured times, a fixed part and a
-//     part per round of the device's slots, linear in K. A last round of
-//     128 x 128 tiles that puts one on each CU takes 0.65 of a full one; the
-//     large tiles' fixed part is a prologue and an epilogue with no other
-//     workgroup to run beside. 4096 x 3072 -> 9216: 192 x 256 123.2 -> 119.7
-//     (256 x 256: 130.9, 128 x 128: 135.1); 4608 x 3072 -> 21504: 256 x 256
-//     306.8 -> 280.8 (128 x 128: 315.4); 8192 x 640 -> 5120: 128 x 128 49.2 ->
-//     42.6 (256 x 256: 43.2).
+//   above: the least time by a fit of the three tiles' measured times over 297
+//     shapes with operands from the cache and from HBM: a fixed part and a part
+//     per round of the device's slots, linear in K, where a last round counts a
+//     part of a full one at once and the rest by how full it is (the clock
+//     rises as CUs fall idle). Its choice is within 0.5% of the best of the
+//     three on average; at 192 x 256 / 256 x 256 / 128 x 128 us: 4096 x 3072 ->
+//     9216 121 / 134 / 140, 4096 x 3072 -> 12288 161 / 148 / 180, 8192 x 640 ->
+//     5120 54.0 / 48.5 / 49.6, 16384 x 640 -> 2560 56.1 / 50.8 / 47.8, 8192 x
+//     1280 -> 2560 40.0 / 44.0 / 40.2, 7904 x 640 -> 1920 27.0 / 22.3 / 20.9.
 // K = 64 (mod 128): 64-byte stages at 128 x 128, 3 workgroups per CU; 8192 x
-// 320 -> 1280 with float32 out 18.4 -> 12.7 us. Only below K = 1024: deeper
-// ones would want the larger tiles of the register-staged kernel.
+// 320 -> 1280 with float32 out 18.4 -> 12.7 us, 16384 x 448 -> 2560 51.3 ->
+// 41.4. Only below K = 1024: at K = 704 it is ahead at every size of 64 to
+// 65536 rows (4096 -> 5120 35.8 -> 31.2), at 832 and 960 ahead (4096 x 960 ->
+// 1280 15.3 -> 13.3) or up to 7% behind (4096 x 960 -> 2560 22.4 -> 24.2, 65536
+// x 960 -> 1280 127 -> 136) by how full the last rounds are; deeper ones want
+// the larger tiles of the register-staged kernel.
 enum DmaPick {
   DMA_NONE = 0,
   DMA_256x256 = DC_GEMM_DMA_256x256,
@@ -1074,11 +1080,14 @@ static DmaPick pick_dma(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
   if (t128 <= cus) return DMA_128x128D;
   if (t128 <= 2 * cus) return DMA_128x128;
   const double k = (double)K;
-  const auto rounds = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
-  const int64_t full = t128 / (2 * cus), rest = t128 % (2 * cus);
-  const double c128 = 1.5 + ((double)full + (rest == 0 ? 0.0 : rest <= cus ? 0.65 : 1.0)) * (3.4 + 0.0080 * k);
-  const double c192 = 5.0 + rounds(tiles(192, 256)) * (2.5 + 0.0112 * k);
-  const double c256 = 6.4 + rounds(tiles(256, 256)) * (4.0 + 0.0135 * k);
+  // t tiles in rounds of `slots`, a last round that is not full counting `part` and up
+  const auto rounds = [](int64_t t, int64_t slots, double part) {
+    const int64_t rest = t % slots;
+    return (double)(t / slots) + (rest ? part + (1.0 - part) * (double)rest / (double)slots : 0.0);
+  };
+  const double c128 = 2.5 + rounds(t128, 2 * cus, 0.40) * (4.1 + 0.0084 * k);
+  const double c192 = 3.2 + rounds(tiles(192, 256), cus, 0.45) * (6.8 + 0.0116 * k);
+  const double c256 = 2.1 + rounds(tiles(256, 256), cus, 0.50) * (10.1 + 0.0133 * k);
   if (c128 <= c192 && c128 <= c256) return DMA_128x128;
   return c192 < c256 ? DMA_192x256 : DMA_256x256;
 }

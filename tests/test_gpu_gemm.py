@@ -146,10 +146,10 @@ def test_short_input(gpu):
 # 256-CU device, and K % 256 for DMA_256x256) and the kernel that runs them,
 # with M, N and K tails among them; the register-staged kernel at each of its
 # four tiles
-TILE_SHAPES = [((4096, 12288, 512), "dma_256x256", "dma_192x256"), ((4608, 3072, 256), "dma_256x256", "dma_128x128"),
+TILE_SHAPES = [((4096, 12288, 512), "dma_256x256", "dma_256x256"), ((4608, 3072, 256), "dma_256x256", "dma_128x128"),
                ((4096, 12288, 272), "256x256", "256x256"), ((4096, 3072, 512), "192x256", "dma_192x256"),
                ((4000, 3000, 272), "192x256", "192x256"), ((512, 3072, 512), "128x128", "dma_64x128"),
-               ((4001, 12200, 768), "dma_256x256", "dma_192x256"), ((512, 12288, 3072), "192x128", "dma_128x128"),
+               ((4001, 12200, 768), "dma_256x256", "dma_256x256"), ((512, 12288, 3072), "192x128", "dma_128x128"),
                ((500, 12200, 336), "192x128", "192x128"), ((500, 3070, 528), "128x128", "128x128"),
                ((2500, 6140, 1024), "dma_256x256", "dma_256x256")]
 
@@ -495,8 +495,9 @@ def test_multi_round_grouped_gemm_bit_exact(gpu, ms, n, k, dtype, bias_dtype):
 DMA_EDGES = [("dma_64x64", [(1, 8, 128), (64, 64, 256), (65, 130, 384), (154, 2560, 512), (129, 513, 128)]),
              ("dma_64x128", [(512, 3071, 640), (500, 3072, 1280), (1000, 2048, 256)]),
              ("dma_128x128_8w", [(1025, 2049, 384), (2048, 1281, 512)]),
-             ("dma_128x128", [(2047, 3840, 128), (2000, 3840, 384), (7904, 1920, 640)]),
-             ("dma_192x256", [(4096, 3072, 1024), (4095, 3001, 384), (2560, 16384, 256), (2500, 16380, 384)]),
+             ("dma_128x128", [(2047, 3840, 128), (2000, 3840, 384), (7904, 1920, 640), (2560, 16384, 256),
+                              (2500, 16380, 384)]),
+             ("dma_192x256", [(4096, 3072, 1024), (4095, 3001, 384)]),
              ("dma_256x256", [(2304, 6144, 1024), (2500, 6140, 1536)]),
              ("dma_128x128_k64", [(1, 4, 64), (130, 260, 192), (8192, 1280, 320), (3000, 1284, 576), (100, 100, 960)]),
              ("128x128", [(257, 300, 1088), (300, 200, 48)])]
