@@ -1130,7 +1130,10 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, int* kslice) {
 //   64 x 64 while it makes 4 slices or more; with 2 or 3 of them the chain
 //     stays long from K = 7680, and a tile of 128 rows takes over, in the order
 //     of the measured best: three slices that fill the CUs; 4 slices (two
-//     workgroups per CU); 64 x 128; 8-wave 128 x 128 up to half the CUs' tiles.
+//     workgroups per CU); 64 x 128; 8-wave 128 x 128 up to half the CUs' tiles,
+//     in two slices from K = 10240 (below, they gain only where the operands
+//     come from HBM: 512 x 8192 -> 3072 28.3 against 30.5 unsplit, but 26.1
+//     against 24.1 from the Infinity Cache).
 // Graph time over operands that no cache holds, fp16 out: the register-staged
 // split / unsplit (or 4 slices of 64 x 64 from K = 8192, where K % 512 == 0) /
 // this rule: 1 x 6144 -> 3072 13.3 / 19.2 / 10.5 us, 64 x 8320 -> 3072 18.4 /
@@ -1139,7 +1142,7 @@ static int splitk_plan(int64_t M, int64_t N, int64_t K, int* kslice) {
 // 48.4 / 55.2 / 45.5. On the lines, unsplit against split: 100 x 4096 -> 3072
 // 10.2 / 10.3 (2), 512 x 5120 -> 1280 12.4 / 13.1 (3), 512 x 5120 -> 3072 21.1
 // / 22.1 (2), 231 x 8192 -> 8192 33.2 / 34.4 (2), 512 x 12288 -> 5120 60.7 /
-// 69.2 (4). Over 848 shapes of up to 640 rows the rule is within 2.2% of the
+// 69.2 (4). Over 848 shapes of up to 640 rows the rule is within 2.3% of the
 // best of all tiles and slices on average, and nowhere over 4% behind what ran
 // before it.
 static int dma_splits(int64_t M, int64_t N, int64_t K, DmaPick* tile, int* kslice) {
@@ -1163,7 +1166,7 @@ static int dma_splits(int64_t M, int64_t N, int64_t K, DmaPick* tile, int* kslic
   else if (s64 == 3 && 10 * s64 * t64 >= 9 * cus && !longest_k) s = 3;
   else if (s64 == 2 && long_k && !(longest_k && s64x128 >= 4 && M <= 512)) s = 4;
   else if (s64x128 >= 3 && K >= 6144) s = s64x128, *tile = DMA_64x128;
-  else if (s128 >= 2 && long_k && 2 * t128 <= cus) s = s128, *tile = DMA_128x128D;
+  else if (s128 >= (longest_k ? 2 : 3) && long_k && 2 * t128 <= cus) s = s128, *tile = DMA_128x128D;
   if (s < 2) return 1;
   const int64_t slice = (K / 128 + s - 1) / s * 128;
   *kslice = (int)slice;

@@ -242,7 +242,8 @@ SPLIT_K = [((512, 3072, 3072), "dma_64x128", 1), ((154, 1280, 2048), "dma_64x64"
            ((1, 5120, 7680), "dma_64x64", 6), ((33, 9000, 7808), "dma_64x64", 3), ((231, 2040, 8320), "dma_64x64", 4),
            ((400, 640, 12416), "dma_64x128", 6), ((100, 3069, 15360), "dma_64x128", 5),
            ((500, 1276, 6272), "dma_64x128", 3), ((512, 3072, 12288), "dma_128x128_8w", 2),
-           ((154, 3069, 7680), "dma_128x128_8w", 4),
+           ((154, 3069, 7680), "dma_128x128_8w", 4), ((300, 3072, 8192), "dma_128x128_8w", 3),
+           ((512, 3072, 8192), "dma_64x128", 1),
            ((154, 640, 4112), "128x128", 7), ((77, 1280, 3088), "128x128", 4), ((300, 520, 2112), "128x128", 4),
            ((77, 640, 2064), "128x128", 4), ((512, 3072, 3088), "128x128", 4)]
 
