@@ -6,8 +6,7 @@ synchronizations, the outputs are overwritten with NaN before each replay
 captured input buffers must reach the next replay.
 
 Covered: the quantize kernel, GEMM tiles of the FLUX step (DMA-fed 128 x 128
-and 64 x 128, register-staged 192 x 128 at the text MLP-up shape),
-split-K with its workspace and epilogue pass, a grouped launch of two layers
+and 64 x 128), split-K with its workspace and epilogue pass on both kernels, a grouped launch of two layers
 on 256 x 256 tiles, the same pair with the gated residual epilogue, and the
 INT8 attention (K statistics, K quantize, attention): the
 DMA-fed kernel with 256-query tiles at the FLUX shape, with 128-query tiles
@@ -28,8 +27,8 @@ from diffucore_amd import _int8, attention_bhld
 pytestmark = pytest.mark.gpu
 
 BF16 = torch.bfloat16
-# (M, K, N): 256 x 256 class, 64 x 128 tiles, the register-staged 192 x 128
-# (FLUX's text MLP up), a ragged one, split-K on the DMA-fed and the
+# (M, K, N): 256 x 256 class, 64 x 128 tiles, 128 x 128 ones (FLUX's text MLP
+# up, class 192 x 128), a ragged one, split-K on the DMA-fed and the
 # register-staged kernel; the last two run as one grouped launch
 # (dc_w8a8_gemm_grouped)
 LINEARS = [(4096, 512, 4096), (512, 3072, 3072), (512, 3072, 12288), (1000, 768, 1280), (512, 12288, 1024),

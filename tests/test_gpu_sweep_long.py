@@ -1,14 +1,14 @@
 """Long seeded sweeps (about a minute on one MI355X).
 
 The same checks as ``tests/test_gpu_sweep.py`` over more random cases, plus
-large shapes that take the DMA-fed kernels, multi-round grids, stream-K
-attention plans and split-K GEMMs:
+large shapes that take the DMA-fed kernels, multi-round grids and stream-K
+attention plans, and few rows over a deep K, which split it:
 
 * W8A8 linear, large: activation codes and scales bit-exact against the
   oracle's quantizer; the int32 products against ``torch._int_mm`` (the
   vendor GEMM the reference's ``int_mm`` calls, ``_int8.py:200-207``) and,
   through the oracle's ``rescale`` (``:313-323``), the fused output bit for
-  bit.
+  bit. The deep ones the same, against float64 products (exact below 2^53).
 * INT8 attention, large: K codes, block scales, key sums and Q codes
   bit-exact against the oracle over the whole input; the output against the
   oracle's restatement on 48 random query rows (each row depends only on its
@@ -51,6 +51,23 @@ def _big_linear_cases(n: int, seed: int):
         bias = [None, dtype, torch.float32][int(rng.integers(0, 3))]
         cases.append((i, M, N, K, group, dtype, bias))
     return cases
+
+
+def _deep_linear_cases(n: int, seed: int):
+    rng = np.random.default_rng(seed)
+    cases = []
+    for i in range(n):
+        group = int(rng.choice([0, 256]))
+        K = int(rng.integers(16, 65)) * 256 if group else int(rng.integers(256, 1025)) * 16
+        M = int(rng.choice([1, 33, 64, 77, 154, 512, int(rng.integers(1, 640))]))
+        N = int(rng.choice([640, 1280, 3072, int(rng.integers(1, 640)) * 8]))
+        dtype = _FLOATS[int(rng.integers(0, 3))]
+        bias = [None, dtype, torch.float32][int(rng.integers(0, 3))]
+        cases.append((i, M, N, K, group, dtype, bias))
+    return cases
+
+
+DEEP_CASES = _deep_linear_cases(32, 424242)
 
 
 def _big_attn_cases(n: int, seed: int):
@@ -112,6 +129,26 @@ def test_linear_long_sweep_large(gpu, i, M, N, K, group, dtype, bias_dtype):
     with torch.no_grad():
         y = layer(xd)
     acc = torch._int_mm(q, layer.weight.t())
+    assert torch.equal(_int8.int_mm(q, layer.weight), acc)
+    b = None if bias_dtype is None else np32(layer.bias)
+    ref = OG.rescale(acc.cpu().numpy(), s_ref, layer.scale.cpu().numpy(), b, DT[dtype])
+    assert np.array_equal(np32(y).view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("i,M,N,K,group,dtype,bias_dtype", DEEP_CASES)
+def test_linear_long_sweep_deep(gpu, i, M, N, K, group, dtype, bias_dtype):
+    kernel, slices = _int8.gemm_kernel(M, N, K)
+    print(f"[long sweep] deep linear {i}: M {M} N {N} K {K} group {group} {DT[dtype]} bias {bias_dtype}: {kernel}, "
+          f"{slices} slices", flush=True)
+    layer, g = _layer(K, N, group, bias_dtype, 8000 + i, gpu)
+    x = _activation(M, K, dtype, g)
+    xd = x.to(gpu)
+    q, _ = _int8.quantize_activation(xd, group)
+    q_ref, s_ref = OQ.quantize_activation(np32(x), group)
+    assert np.array_equal(q.cpu().numpy(), q_ref)
+    with torch.no_grad():
+        y = layer(xd)
+    acc = (q.double() @ layer.weight.double().t()).to(torch.int32)
     assert torch.equal(_int8.int_mm(q, layer.weight), acc)
     b = None if bias_dtype is None else np32(layer.bias)
     ref = OG.rescale(acc.cpu().numpy(), s_ref, layer.scale.cpu().numpy(), b, DT[dtype])
